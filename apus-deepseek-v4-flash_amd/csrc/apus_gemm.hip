@@ -1529,11 +1529,14 @@ __global__ __launch_bounds__(256) void apus_gemm_narrow_kernel(ApusGemmArgs args
     uint8_t *wring = lring + (AL ? wave * PD * SLOT : 0);
     const unsigned wbase = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)wring);
     const uint8_t *bp = ent.w + ((size_t)tile * NQ * 128 + lane) * 16;
-    const uint8_t *wsp = ent.ws + (size_t)(tile >> 3) * NQ + q0;     /* 128 x 128 tile scales */
+    /* 128 x 128 tile scales, four to a word. The address is uniform, so these
+     * are scalar loads, which drop an address's two low bits: waves whose run
+     * starts inside a word (K = 1024: two groups a wave) shift it into place */
+    const uint8_t *wsp = ent.ws + (size_t)(tile >> 3) * NQ + (q0 & ~3);
     unsigned sbw[(NG + 3) / 4];
 #pragma unroll
     for (int i = 0; i < (NG + 3) / 4; ++i)
-        sbw[i] = __builtin_amdgcn_readfirstlane(apus_gld<unsigned>(wsp + 4 * i));
+        sbw[i] = __builtin_amdgcn_readfirstlane(apus_gld<unsigned>(wsp + 4 * i)) >> (8 * (q0 & 3));
     struct Grp { apus_v4u b0, b1, a0[AL ? 1 : TM], a1[AL ? 1 : TM]; float s[TM]; };
     auto load = [&](Grp &f, int i) {
         const int q = q0 + i;
