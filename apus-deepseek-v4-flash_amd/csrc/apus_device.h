@@ -132,6 +132,21 @@ __device__ __forceinline__ void apus_lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
+typedef __attribute__((address_space(3))) void apus_lds_void;
+typedef const __attribute__((address_space(1))) void apus_gbl_void;
+/* 16 (or 4) bytes per lane from global memory straight into LDS at
+ * lds + 16 * lane (4 * lane); lds must be the same in every lane */
+__device__ __forceinline__ void apus_g2lds16(const void *g, unsigned lds) {
+    __builtin_amdgcn_global_load_lds((apus_gbl_void *)g,
+                                     (apus_lds_void *)(uintptr_t)__builtin_amdgcn_readfirstlane(lds), 16, 0, 0);
+}
+__device__ __forceinline__ void apus_g2lds4(const void *g, unsigned lds) {
+    __builtin_amdgcn_global_load_lds((apus_gbl_void *)g,
+                                     (apus_lds_void *)(uintptr_t)__builtin_amdgcn_readfirstlane(lds), 4, 0, 0);
+}
+template <int N>
+__device__ __forceinline__ void apus_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
 /* 16-byte chunk slot of chunk c of a 128-byte activation row staged in LDS:
  * c ^ apus_row_swz(row). A fragment read (ds_read_b128, lane (r, g) reading
  * chunk g or 4 + g of row r, 16 rows) is then conflict-free on gfx950:

@@ -1336,21 +1336,6 @@ __global__ __launch_bounds__(64 * NW) void apus_gemm_tile_kernel(ApusGemmArgs ar
 #ifndef APUS_PRE_LDS_NST
 #define APUS_PRE_LDS_NST 3
 #endif
-typedef __attribute__((address_space(3))) void apus_lds_void;
-typedef const __attribute__((address_space(1))) void apus_gbl_void;
-/* 16 (or 4) bytes per lane from global memory straight into LDS at
- * lds + 16 * lane (4 * lane); lds must be the same in every lane */
-__device__ __forceinline__ void apus_g2lds16(const void *g, unsigned lds) {
-    __builtin_amdgcn_global_load_lds((apus_gbl_void *)g,
-                                     (apus_lds_void *)(uintptr_t)__builtin_amdgcn_readfirstlane(lds), 16, 0, 0);
-}
-__device__ __forceinline__ void apus_g2lds4(const void *g, unsigned lds) {
-    __builtin_amdgcn_global_load_lds((apus_gbl_void *)g,
-                                     (apus_lds_void *)(uintptr_t)__builtin_amdgcn_readfirstlane(lds), 4, 0, 0);
-}
-template <int N>
-__device__ __forceinline__ void apus_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
 template <int NQ>
 __global__ __launch_bounds__(512, 1) void apus_gemm_lds_kernel(ApusGemmArgs args) {
     extern __shared__ __align__(16) uint8_t lds[];

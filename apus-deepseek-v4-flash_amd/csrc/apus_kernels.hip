@@ -686,6 +686,304 @@ __global__ __launch_bounds__(256) void apus_head_kernel(const uint16_t *__restri
     }
 }
 
+/* ------------------------------------------- plain-weight GEMM (M > 8) */
+
+/* The same linears over more than 8 rows of x (prompts, decode batches: the
+ * output projection's BF16 groups, the router gate, compressor weights): an
+ * MFMA kernel, because apus_wgemv_kernel re-reads the weights for every 8
+ * rows and runs on the vector units. One workgroup of NW waves owns TM 16-row
+ * x tiles by TN 16-row weight tiles; its waves split K in interleaved
+ * 32-element steps, each bringing its own operands global -> LDS into a
+ * private ring PD steps deep (no barrier in the loop; a slot is refilled as
+ * soon as its fragments are in registers), and the partial tiles meet in LDS,
+ * added in a fixed tree. Fragments loaded straight from global memory instead
+ * (16 rows a load: a tag lookup per lane) ran 37 us where this runs 24.6.
+ *
+ * Products are exact in fp32 and sums are fp32:
+ * - BF16 weights, x rounded to BF16 (flag 1): one BF16 MFMA;
+ * - BF16 weights, fp32 x: three BF16 pieces that add up to x exactly, one
+ *   MFMA each;
+ * - FP32 weights: the fp32 MFMA (16x16x4).
+ * Chains are short, for accuracy: BF16 ones are flushed into a second
+ * accumulator every FL steps, the small pieces in a chain of their own, FP32
+ * ones are 8 products long. Error against 64 bits at K = 1000 / 2048 / 4096:
+ * BF16 0.80 / 0.85 / 0.90e-7, FP32 0.91 / 0.99 / 1.12e-7, where
+ * apus_wgemv_kernel's lane chains give 0.99 / 1.23 / 1.59e-7.
+ *
+ * 512 x 1024 x 4096: BF16 weights 137 -> 21-25 us (175-200 TFLOP/s), FP32
+ * weights 132 -> 53 us (half the fp32 MFMA rate). Bound by the L2 -> CU stream of
+ * both operands (1 MB a CU) and the splitting of x on the vector units. */
+typedef __bf16 apus_v8bf __attribute__((ext_vector_type(8)));
+
+/* BF16 pieces of 8 fp32 values, nearest-even (one packed conversion per two
+ * values): P = 1 the rounded values, P = 3 x = hi + mid + lo exactly. With a
+ * non-finite value among them (a wave-uniform test) hi is cut from the bits and
+ * the rest is zero for it, so that it stays what it is. */
+typedef __bf16 apus_v2bf __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t apus_cvt_pk_bf16(float a, float b) {
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), apus_v2bf));
+}
+template <int P>
+__device__ __forceinline__ void apus_bf16_pieces(const float (&v)[8], apus_v8bf (&out)[P]) {
+    uint32_t q[P][4];
+    bool special = false;
+    if constexpr (P == 3) {
+        uint32_t m = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) m = max(m, __float_as_uint(v[i]) & 0x7fffffffu);
+        /* from 0x7f7f8000 on the rounding would give an infinity */
+        special = __any(m >= 0x7f7f8000u);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = v[2 * i], b = v[2 * i + 1];
+        q[0][i] = apus_cvt_pk_bf16(a, b);
+        if constexpr (P == 3) {
+            const float a1 = a - __uint_as_float(q[0][i] << 16), b1 = b - __uint_as_float(q[0][i] & 0xffff0000u);
+            q[1][i] = apus_cvt_pk_bf16(a1, b1);
+            q[2][i] = apus_cvt_pk_bf16(a1 - __uint_as_float(q[1][i] << 16),
+                                       b1 - __uint_as_float(q[1][i] & 0xffff0000u));
+        }
+    }
+    if constexpr (P == 3) {
+        if (special) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                uint32_t c[3][2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float x = v[2 * i + h];
+                    const uint32_t u = __float_as_uint(x);
+                    c[0][h] = x != x ? u | 0x400000u : u & 0xffff0000u;
+                    const float r = (u & 0x7f800000u) == 0x7f800000u ? 0.0f : x - __uint_as_float(c[0][h]);
+                    c[1][h] = __float_as_uint(r) & 0xffff0000u;
+                    c[2][h] = __float_as_uint(r - __uint_as_float(c[1][h]));
+                }
+#pragma unroll
+                for (int p = 0; p < 3; ++p) q[p][i] = (c[p][0] >> 16) | (c[p][1] & 0xffff0000u);
+            }
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+        out[p] = __builtin_bit_cast(apus_v8bf, apus_v4u{q[p][0], q[p][1], q[p][2], q[p][3]});
+}
+
+template <bool WB, int P, int TM, int TN, int PD, int NW>
+__global__ __launch_bounds__(64 * NW) void apus_wgemm_kernel(const void *__restrict__ w,
+                                                         const float *__restrict__ x,
+                                                         float *__restrict__ out, int M, int K, int O,
+                                                         int flags) {
+    constexpr int EB = WB ? 2 : 4, FL = P == 1 ? 2 : 4;
+    constexpr int XB = TM * 2048, WBY = TN * 512 * EB, STB = XB + WBY;   /* bytes of a step: x, weights */
+    constexpr int NLX = XB / 1024, NL = STB / 1024;                      /* loads of a step */
+    static_assert(PD <= 4 && (PD - 1) * NL < 64, "vmcnt");
+    extern __shared__ __align__(16) uint8_t wlds[];                      /* NW x PD x STB; then the sums */
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * (16 * TN), m0 = blockIdx.y * (16 * TM);
+    uint8_t *ring = wlds + wave * PD * STB;
+    const unsigned rbase = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)ring);
+    /* load u of a step brings 1 KB: eight 128-byte rows (32 fp32 elements),
+     * LDS slot p of row i holding 16-byte chunk p ^ (i & 7), or sixteen 64-byte
+     * rows (32 BF16 elements), slot p holding chunk p ^ ((i >> 2) & 3): fragment
+     * reads are then free of bank conflicts. ke: the lane's first element */
+    const uint8_t *src[NL];
+    int ke[NL];
+#pragma unroll
+    for (int u = 0; u < NL; ++u) {
+        const bool isx = u < NLX;
+        if (isx || !WB) {
+            const int i = 8 * (isx ? u : u - NLX) + (lane >> 3), c = (lane & 7) ^ (i & 7);
+            const size_t row = isx ? min(m0 + i, M - 1) : min(n0 + i, O - 1);
+            ke[u] = 4 * c;
+            src[u] = (isx ? (const uint8_t *)x : (const uint8_t *)w) + row * K * 4 + 16 * c;
+        } else {
+            const int i = 16 * (u - NLX) + (lane >> 2), c = (lane & 3) ^ ((i >> 2) & 3);
+            ke[u] = 8 * c;
+            src[u] = (const uint8_t *)w + (size_t)min(n0 + i, O - 1) * K * 2 + 16 * c;
+        }
+    }
+    /* step s: elements [32 s, 32 s + 32); past K the row's first chunk is
+     * read instead (in bounds; cleared at the fragment) */
+    auto issue = [&](int s, int slot) {
+        if (32 * s + 32 <= K) {
+#pragma unroll
+            for (int u = 0; u < NL; ++u)
+                apus_g2lds16(src[u] + (size_t)s * (WB && u >= NLX ? 64 : 128), rbase + slot * STB + u * 1024);
+        } else {
+#pragma unroll
+            for (int u = 0; u < NL; ++u) {
+                const int eb = WB && u >= NLX ? 2 : 4;
+                const ptrdiff_t off = 32 * s + ke[u] < K ? (ptrdiff_t)s * 32 * eb : -(ptrdiff_t)ke[u] * eb;
+                apus_g2lds16(src[u] + off, rbase + slot * STB + u * 1024);
+            }
+        }
+    };
+    /* chains: BF16 [0] of the (first) pieces, [1] of the small pieces */
+    apus_v4f acc[2][TM][TN] = {}, tot[TM][TN] = {};
+    const int nst = (K + 31) >> 5;
+    const int own = wave < nst ? (nst - wave + NW - 1) / NW : 0;         /* this wave's steps */
+#pragma unroll
+    for (int d = 0; d < PD; ++d)
+        if (d < own) issue(wave + d * NW, d);
+    for (int c = 0; c < own; ++c) {
+        const int later = min(own - 1 - c, PD - 1);                      /* steps in flight behind this one */
+        if (PD > 3 && later >= 3) apus_wait_vm<3 * NL>();
+        else if (PD > 2 && later == 2) apus_wait_vm<2 * NL>();
+        else if (PD > 1 && later == 1) apus_wait_vm<NL>();
+        else apus_wait_vm<0>();
+        const int s = wave + c * NW;
+        const uint8_t *stg = ring + (c % PD) * STB;
+        /* the step's fragments to registers, then its slot is refilled */
+        float4 fa[TM][2];
+        apus_v4u fb[TN][WB ? 1 : 2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                fa[i][h] = *reinterpret_cast<const float4 *>(
+                    stg + (16 * i + r) * 128 + (((WB ? 2 * g + h : 4 * h + g) ^ (r & 7)) << 4));
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            if constexpr (WB) {
+                fb[j][0] = *reinterpret_cast<const apus_v4u *>(stg + XB + (16 * j + r) * 64 + ((g ^ ((r >> 2) & 3)) << 4));
+            } else {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    fb[j][h] = *reinterpret_cast<const apus_v4u *>(stg + XB + (16 * j + r) * 128 +
+                                                                   (((4 * h + g) ^ (r & 7)) << 4));
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (c + PD < own) issue(wave + (c + PD) * NW, c % PD);
+        if (32 * s + 32 > K) {                                           /* elements past K */
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const bool in = 32 * s + (WB ? 8 * g : 16 * h + 4 * g) < K;
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    if (!in) fa[i][h] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    if (!in) fb[j][WB ? 0 : h] = apus_v4u{0u, 0u, 0u, 0u};
+            }
+        }
+        if constexpr (WB) {
+            apus_v8bf a[TM][P];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const float e[8] = {fa[i][0].x, fa[i][0].y, fa[i][0].z, fa[i][0].w,
+                                    fa[i][1].x, fa[i][1].y, fa[i][1].z, fa[i][1].w};
+                apus_bf16_pieces<P>(e, a[i]);
+            }
+#pragma unroll
+            for (int p = P - 1; p >= 0; --p)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[p > 0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            a[i][p], __builtin_bit_cast(apus_v8bf, fb[j][0]), acc[p > 0][i][j], 0, 0, 0);
+        } else {
+            apus_v4f ah[4][TM][TN] = {};                                 /* chains of 8 */
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (flags & 1) {
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) {
+                        float4 &v = fa[i][h];
+                        v.x = apus_bf16_rne(v.x); v.y = apus_bf16_rne(v.y);
+                        v.z = apus_bf16_rne(v.z); v.w = apus_bf16_rne(v.w);
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) {
+                        const float4 &v = fa[i][h];
+                        const float e = q == 0 ? v.x : q == 1 ? v.y : q == 2 ? v.z : v.w;
+#pragma unroll
+                        for (int j = 0; j < TN; ++j)
+                            ah[2 * h + (q >> 1)][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                e, __uint_as_float(fb[j][WB ? 0 : h][q]), ah[2 * h + (q >> 1)][i][j], 0, 0, 0);
+                    }
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) tot[i][j] += (ah[0][i][j] + ah[1][i][j]) + (ah[2][i][j] + ah[3][i][j]);
+        }
+        if (WB && (c + 1) % FL == 0) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    tot[i][j] += P > 1 ? acc[0][i][j] + acc[1][i][j] : acc[0][i][j];
+                    acc[0][i][j] = acc[1][i][j] = apus_v4f{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    }
+    __syncthreads();                                                     /* the rings become the sums' space */
+    apus_v4f *red = reinterpret_cast<apus_v4f *>(wlds);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) red[(wave * TM * TN + i * TN + j) * 64 + lane] = tot[i][j] + (acc[0][i][j] + acc[1][i][j]);
+    __syncthreads();
+    /* lane holds D[4g + q][r]: x row 16 i + 4 g + q, weight row 16 j + r */
+    for (int e = threadIdx.x; e < TM * TN * 64; e += 64 * NW) {
+        const int tile = e >> 6, l = e & 63;
+        apus_v4f p[NW];
+#pragma unroll
+        for (int k = 0; k < NW; ++k) p[k] = red[k * TM * TN * 64 + e];
+#pragma unroll
+        for (int d = 1; d < NW; d *= 2)
+#pragma unroll
+            for (int k = 0; k < NW; k += 2 * d) p[k] += p[k + d];
+        const apus_v4f v = p[0];
+        const int o = n0 + 16 * (tile % TN) + (l & 15), m = m0 + 16 * (tile / TN) + 4 * (l >> 4);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (o < O && m + q < M) out[(size_t)(m + q) * O + o] = (flags & 2) ? apus_bf16_rne(v[q]) : v[q];
+    }
+}
+
+template <bool WB, int P, int TM, int TN, int PD, int NW>
+bool apus_launch_wgemm_tile(const void *w, const float *x, float *out, int M, int K, int O, int flags,
+                            hipStream_t st) {
+    constexpr int ring = NW * PD * (TM * 2048 + TN * 512 * (WB ? 2 : 4)), sums = NW * TM * TN * 1024;
+    constexpr int lds = ring > sums ? ring : sums;
+    static const hipError_t attr = hipFuncSetAttribute(
+        reinterpret_cast<const void *>(&apus_wgemm_kernel<WB, P, TM, TN, PD, NW>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return false;
+    hipLaunchKernelGGL((apus_wgemm_kernel<WB, P, TM, TN, PD, NW>),
+                       dim3((O + 16 * TN - 1) / (16 * TN), (M + 16 * TM - 1) / (16 * TM)), dim3(64 * NW), lds, st, w, x,
+                       out, M, K, O, flags);
+    return true;
+}
+
+template <bool WB, int P>
+bool apus_launch_wgemm(const void *w, const float *x, float *out, int M, int K, int O, int flags,
+                       hipStream_t st) {
+    /* the largest tile that still gives most CUs a workgroup: a workgroup's
+     * time is its own stream and conversions, so idle CUs cost more than
+     * re-reads (BF16, K = 4096: 512 x 1024, 256 / 512 workgroups of 32 x 64 /
+     * 32 x 32, 24.6 / 35.8 us; 254 x 1000, 128 / 256 workgroups, 18.6 / 12.2;
+     * 20 x 1024, 16 x 32 tiles 10.0, 32 x 32 13.9; FP32 512 x 256, 128 / 256
+     * workgroups of 32 x 32 / 16 x 32, 29.7 / 17.6) */
+    auto fills = [&](int tm, int tn) {
+        return (size_t)((M + 16 * tm - 1) / (16 * tm)) * ((O + 16 * tn - 1) / (16 * tn)) >= 192;
+    };
+    if constexpr (WB) {
+        if (fills(2, 4)) return apus_launch_wgemm_tile<WB, P, 2, 4, 2, 8>(w, x, out, M, K, O, flags, st);
+    }
+    if (fills(2, 2)) return apus_launch_wgemm_tile<WB, P, 2, 2, 2, 8>(w, x, out, M, K, O, flags, st);
+    return apus_launch_wgemm_tile<WB, P, 1, 2, 3, 8>(w, x, out, M, K, O, flags, st);
+}
+
 hipError_t apus_launch_wgemv(const void *w, const float *x, float *out, int M, int K, int O,
                              int flags, hipStream_t st) {
     if (M <= 0 || O <= 0) return hipSuccess;
@@ -709,6 +1007,13 @@ hipError_t apus_launch_wgemv(const void *w, const float *x, float *out, int M, i
         if (flags & 4) hipLaunchKernelGGL((apus_wgemv_kernel<true, 1>), dim3(gx), block, 0, st, w, x, out, M, K, O, flags);
         else           hipLaunchKernelGGL((apus_wgemv_kernel<false, 1>), dim3(gx), block, 0, st, w, x, out, M, K, O, flags);
         return hipGetLastError();
+    }
+    /* its 16-byte loads go straight to LDS: rows have to be 16-byte aligned */
+    if (M > 8 && ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15) == 0) {
+        const bool ok = !(flags & 4) ? apus_launch_wgemm<false, 1>(w, x, out, M, K, O, flags, st)
+                      : (flags & 1)  ? apus_launch_wgemm<true, 1>(w, x, out, M, K, O, flags, st)
+                                     : apus_launch_wgemm<true, 3>(w, x, out, M, K, O, flags, st);
+        if (ok) return hipGetLastError();
     }
     const dim3 grid(gx, (M + 7) / 8);
     if (flags & 4) hipLaunchKernelGGL((apus_wgemv_kernel<true, 8>), grid, block, 0, st, w, x, out, M, K, O, flags);

@@ -101,3 +101,56 @@ def test_head_gemv_full_size(hip, oracle):
     rows = np.unique(np.concatenate([np.arange(256), np.arange(O - 256, O),
                                      rng.choice(O, 1024, replace=False)]))
     _check(got[None, rows], oracle, w[rows], x[None, :], 4)
+
+
+@pytest.mark.parametrize("M,K,O,flags", [(9, 8, 1, 0), (17, 40, 33, 4), (16, 1000, 77, 7), (33, 264, 65, 6),
+                                         (40, 4096, 64, 0), (100, 1032, 200, 3), (65, 2048, 130, 4),
+                                         (300, 1000, 700, 5), (500, 520, 1000, 4), (513, 72, 500, 0),
+                                         (600, 96, 1025, 6)])
+def test_many_rows(hip, oracle, rng, M, K, O, flags):
+    """More than 8 rows: the matrix-core kernel's three tile sizes, at partial
+    row, weight and K tiles, for every operand form."""
+    w, x = _data(rng, M, K, O, flags & 4)
+    _check(hip.f32_linear(w, x, flags), oracle, w, x, flags)
+
+
+@pytest.mark.parametrize("flags", [0, 3, 4, 5])
+def test_many_rows_non_finite(hip, rng, flags):
+    """Infinities, NaNs and values next to the largest: a 24-row call has them
+    where three 8-row calls (the vector kernel) do, and the other values agree
+    (1e-5 of the row's largest: fp32 sums in another order; one BF16 step)."""
+    M, K, O = 24, 200, 40
+    w, x = _data(rng, M, K, O, flags & 4)
+    x[1, 7], x[5, 0], x[9, 33] = np.inf, -np.inf, np.nan
+    x[12, 11], x[13, 12] = np.float32(3.4e38), np.finfo(np.float32).max
+    x[20, 3], x[20, 4] = np.inf, -np.inf
+    L = hip.lib()
+    dw, dx = hip.DevBuf.from_array(w), hip.DevBuf.from_array(x)
+    outs = []
+    for rows in (24, 8):
+        do = hip.DevBuf(M * O * 4)
+        for m in range(0, M, rows):
+            hip._check(L.apus_hip_wlinear_dev(dw.ptr, dx.ptr + m * K * 4, do.ptr + m * O * 4, rows, K, O,
+                                              flags), "wlinear")
+        hip._check(L.apus_hip_synchronize(), "sync")
+        outs.append(do.to_array(np.float32, (M, O)))
+    a, b = (v.astype(np.float64) for v in outs)
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
+    assert np.array_equal(a[np.isinf(a)], b[np.isinf(b)])
+    fin = np.isfinite(a)
+    scale = np.where(fin, np.abs(b), 0).max(1, keepdims=True) + 1e-30
+    d = np.abs(np.where(fin, a, 0) - np.where(fin, b, 0))
+    assert (d <= (2.0 ** -7 if flags & 2 else 1e-5) * scale).all()
+
+
+def test_many_rows_unaligned(hip, oracle, rng):
+    """Rows that are not 16-byte aligned keep the vector kernel."""
+    M, K, O = 20, 64, 24
+    w, x = _data(rng, M, K, O, False)
+    L = hip.lib()
+    dw = hip.DevBuf.from_array(w)
+    dx = hip.DevBuf.from_array(np.concatenate([np.zeros(1, np.float32), x.ravel()]))
+    do = hip.DevBuf(M * O * 4)
+    hip._check(L.apus_hip_wlinear_dev(dw.ptr, dx.ptr + 4, do.ptr, M, K, O, 0), "wlinear")
+    hip._check(L.apus_hip_synchronize(), "sync")
+    _check(do.to_array(np.float32, (M, O)), oracle, w, x, 0)
