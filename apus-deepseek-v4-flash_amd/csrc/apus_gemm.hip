@@ -30,6 +30,8 @@
 #include "apus_device.h"
 #include "apus_internal.h"
 
+#include <type_traits>
+
 /*
  * Tiling. A workgroup owns 16 consecutive weight rows (the 16 MFMA columns)
  * of one entry and all of that entry's rows (tokens) in tiles of 16. The
@@ -1310,156 +1312,353 @@ __global__ __launch_bounds__(64 * NW) void apus_gemm_tile_kernel(ApusGemmArgs ar
     }
 }
 
-/*
- * LDS tile schedule for dense FP8 GEMMs with more than 8 rows on MFMA-tiled
- * weights (e.g. a 512-token projection): the same 64 x 128 output tile and
- * the same accumulation chain per output (one chain over the 128-groups in
- * order) as apus_gemm_tile_kernel, so the two give identical bits, but both
- * operands travel global -> LDS directly (global_load_lds_dwordx4, no
- * register staging) through NST stages of one 128-group each, read by 8
- * waves (4 x 2, each 16 tokens x 64 weight rows). Per stage: 8 loads of 8
- * whole activation rows (each row's 16-byte chunks XOR-swizzled by the row
- * so the fragment reads are conflict-free) and 16 loads of 1 KB weight
- * fragments (the tiled layout is the MFMA operand order), 3 per wave; the
- * activation scales of every group go to LDS once, up front. Workgroup b
- * takes tile (b & 7) * (tiles / 8) + (b >> 3) when tiles % 8 == 0, so each
- * XCD (workgroups are dealt to the 8 XCDs round robin) works on one band of
- * weight-row blocks and every token block: its weight bytes come from HBM
- * once into that XCD's L2. Measured on gfx950 at M = 512, O = K = 4096 (a
- * fresh weight copy per launch): 17.7 us against 20.6 us for the register-
- * ring tile schedule; 3 / 4 / 5 stages 18.1 / 17.7 / 18.0 us; staging the
- * output through LDS for whole-row stores 18.1; 256 x 128 tiles split over
- * K in 2 or 4 (partners on one XCD, partial sums through L2) 20.9-25.5 us:
- * the partial sums' traffic costs more than the operand bytes they save.
- */
-#define APUS_LT_NST 4
 #ifndef APUS_PRE_LDS_NST
 #define APUS_PRE_LDS_NST 3
 #endif
-template <int NQ>
-__global__ __launch_bounds__(512, 1) void apus_gemm_lds_kernel(ApusGemmArgs args) {
-    extern __shared__ __align__(16) uint8_t lds[];
-    constexpr int NST = APUS_LT_NST < NQ ? APUS_LT_NST : NQ;
-    constexpr int K = NQ * 128;
-    constexpr int BM = 64, AB = BM * 128, STB = AB + 128 * 128;
-    constexpr int LA = BM / 8, LPW = (LA + 16) / 8;
-    constexpr int SI = NQ;                     /* scale loads: one per group (64 rows) */
-    static_assert(SI % 8 == 0, "scale loads");
-    const ApusGemmEnt ent = args.ent0;
-    float *lsc = reinterpret_cast<float *>(lds + NST * STB);     /* [q][64 rows] fp32 */
-    const int M = ent.M;
-    const int MT = (M + BM - 1) / BM, tiles = MT * (args.O >> 7);
-    const int b = blockIdx.x;
-    const int t = (tiles & 7) == 0 ? (b & 7) * (tiles >> 3) + (b >> 3) : b;
-    const int mb = t % MT, nb = t / MT;
-    const int m0 = mb * BM, n0 = nb * 128;
+
+/*
+ * Block schedule: the K loop of the large-tile GEMMs. A workgroup of WM x WN
+ * waves owns BM activation rows x BN weight rows; each wave BM / WM x BN / WN
+ * of them. Both operands travel global -> LDS (global_load_lds_dwordx4)
+ * through NST stages of one 128-group (activations: 8 whole 128-byte rows a
+ * load, 16-byte chunks XOR-swizzled by row; weights: 1 KB fragments of the
+ * tiled layout), and from LDS into a second set of fragment registers one
+ * step ahead of the MFMAs, so a slot is free for its next stage as soon as
+ * the barrier after that read. Scales come per four groups (16 bytes a row),
+ * in a ring of two. Nothing in the loop but these loads uses vmcnt: mixed with
+ * loads into registers, the compiler would drain all of them at each use.
+ * The weights are the MFMA's first operand, so a lane ends up with four
+ * consecutive outputs of one row. Every output is one chain over the
+ * 128-groups in order, as in the smaller tiles (identical bits); with FOLD,
+ * four chains over the quarters of K, added in order.
+ */
+template <int WF, int NQ_, int BM_, int BN_, int WM_, int WN_, int NST_, bool FOLD_ = false>
+struct ApusBlk {
+    static constexpr int NQ = NQ_, BM = BM_, BN = BN_, WM = WM_, WN = WN_, NST = NST_, NW = WM * WN;
+    static constexpr bool FP4 = WF == APUS_W_FP4, FOLD = FOLD_;
+    static constexpr int TM = BM / 16 / WM, TN = BN / 16 / WN, K = NQ * 128;
+    static constexpr int FB = FP4 ? 1024 : 2048;             /* bytes of a weight fragment */
+    static constexpr int AB = BM * 128, STB = AB + BN / 16 * FB;
+    static constexpr int LA = BM / 8, LPW = STB / 1024 / NW; /* loads of a stage: activations; per wave */
+    static constexpr int SI = BM / 64 + (FP4 ? BN / 64 : 0), SPW = (SI + NW - 1) / NW;
+    static constexpr int SB = SI * 1024;                     /* bytes of a scale block (four groups) */
+    static constexpr int LDS = NST * STB + 2 * SB;
+    static_assert(STB / 1024 % NW == 0 && NST >= 2 && NST <= 4 && NQ % 4 == 0 && BM % 64 == 0 && BN % 64 == 0 &&
+                      LDS <= 160 * 1024,
+                  "block shape");
+    /* loads that a wave issues for stage q */
+    static constexpr int loads(int q) { return LPW + (q % 4 == 0 ? SPW : 0); }
+    /* its loads in flight behind stage q when stages up to `last` are issued */
+    static constexpr int behind(int q, int last) {
+        int n = 0;
+        for (int i = q + 1; i <= last; ++i) n += loads(i);
+        return n;
+    }
+};
+
+/* row(i): activation row of the block's row i (any valid row past the end; row *
+ * K below 4 GiB);
+ * wt(t), wst(t): the weight bytes of the block's 16-row tile t and, for FP4,
+ * its scale bytes (tiled layout); sbw(q): FP8, the tile scale of group q for
+ * this wave's columns. acc[i][t]: weight tile i, token tile t of the wave. */
+template <class B, class Row, class Wt, class Wst, class Sbw>
+__device__ __forceinline__ void apus_block_loop(uint8_t *lds, const uint8_t *acodes, const float *ascale, Row row,
+                                                Wt wt, Wst wst, Sbw sbw, apus_v4f (&acc)[B::TN][B::TM]) {
+    constexpr int NQ = B::NQ, NST = B::NST, STB = B::STB, AB = B::AB, TM = B::TM, TN = B::TN;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, g = lane >> 4;
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / B::WN, wn = wave % B::WN;
     const unsigned lbase = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds);
-    /* this wave's loads of a stage: activation instructions ii < LA (8 rows
-     * each: lane -> row 8 ii + lane / 8, LDS slot lane % 8 holding 16-byte
-     * chunk (lane % 8) ^ swizzle(row)), then weight fragments */
-    const uint8_t *src[LPW];
-    unsigned dst[LPW], qs[LPW];
+    /* load sources: a uniform base and a 32-bit lane offset */
+    const uint8_t *sbase[B::LPW];
+    unsigned voff[B::LPW];
 #pragma unroll
-    for (int u = 0; u < LPW; ++u) {
-        const int ii = wave * LPW + u;
-        if (ii < LA) {
-            const int lr = 8 * ii + (lane >> 3), p = lane & 7;
-            const int row = ent.a0 + (m0 + lr < M ? m0 + lr : M - 1);
-            const int sw = apus_row_swz(lr);
-            src[u] = args.acodes + (size_t)row * K + (p ^ sw) * 16;
-            dst[u] = ii * 1024;
-            qs[u] = 128;
+    for (int u = 0; u < B::LPW; ++u) {
+        const int ii = wave * B::LPW + u;
+        if (ii < B::LA) {
+            const int lr = 8 * ii + (lane >> 3);
+            sbase[u] = acodes;
+            voff[u] = (unsigned)row(lr) * (unsigned)B::K + (unsigned)(((lane & 7) ^ apus_row_swz(lr)) * 16);
         } else {
-            const int f = (ii - LA) >> 1, h = (ii - LA) & 1;
-            src[u] = ent.w + ((size_t)((n0 >> 4) + f) * NQ) * 2048 + h * 1024 + lane * 16;
-            dst[u] = AB + f * 2048 + h * 1024;
-            qs[u] = 2048;
+            const int f = ii - B::LA;
+            sbase[u] = B::FP4 ? wt(f) : wt(f >> 1) + (f & 1) * 1024;
+            voff[u] = lane * 16;
         }
     }
-    auto issue = [&](int q, int slot) {
+    const uint8_t *ssrc[B::SPW];
+    unsigned sdst[B::SPW], sstep[B::SPW];
 #pragma unroll
-        for (int u = 0; u < LPW; ++u) apus_g2lds16(src[u] + q * qs[u], lbase + slot * STB + dst[u]);
-    };
-#pragma unroll
-    for (int u = 0; u < SI / 8; ++u) {
-        const int q = wave * (SI / 8) + u;
-        const int row = ent.a0 + (m0 + lane < M ? m0 + lane : M - 1);
-        apus_g2lds4(args.ascale + (size_t)row * NQ + q, lbase + NST * STB + q * BM * 4);
+    for (int u = 0; u < B::SPW; ++u) {
+        const int ii = (wave * B::SPW + u) % B::SI;          /* spare waves repeat a load */
+        if (ii < B::BM / 64) {
+            ssrc[u] = reinterpret_cast<const uint8_t *>(ascale + (size_t)row(64 * ii + lane) * NQ);
+            sstep[u] = 16;
+        } else {
+            const int t = 4 * (ii - B::BM / 64) + (lane >> 4);
+            ssrc[u] = wst(t) + (lane & 15) * 16;
+            sstep[u] = 256;
+        }
+        sdst[u] = NST * STB + ii * 1024;
     }
+    auto issue = [&](int q, int slot, bool sc) {
 #pragma unroll
-    for (int st = 0; st < NST; ++st) issue(st, st);
-    const uint8_t *wsp = ent.ws + (size_t)nb * NQ;     /* 128 x 128 tile scales of this block */
-    unsigned sbw[NQ / 4];
+        for (int u = 0; u < B::LPW; ++u) {
+            const int qs = wave * B::LPW + u < B::LA ? 128 : B::FB;
+            apus_g2lds16(sbase[u] + (size_t)q * qs + voff[u], lbase + slot * STB + (wave * B::LPW + u) * 1024);
+        }
+        if (sc) {
 #pragma unroll
-    for (int i = 0; i < NQ / 4; ++i) sbw[i] = __builtin_amdgcn_readfirstlane(apus_gld<unsigned>(wsp + 4 * i));
-
-    apus_v4f acc[4];
+            for (int u = 0; u < B::SPW; ++u)
+                apus_g2lds16(ssrc[u] + (size_t)(q >> 2) * sstep[u], lbase + sdst[u] + ((q >> 2) & 1) * B::SB);
+        }
+    };
+    struct Frag { apus_v8i w[TN], a[TM]; int sw[TN]; float sa[TM]; };
+    auto read = [&](Frag &f, int q, int slot, int qb) {      /* qb: q & 3, a constant */
+        const uint8_t *stg = lds + slot * STB;
+        const uint8_t *sc = lds + NST * STB + ((q >> 2) & 1) * B::SB;
+        const int sw = apus_row_swz(r);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = apus_v4f{0.f, 0.f, 0.f, 0.f};
-    struct Frag { apus_v8i a, b[4]; int sa; };
-    const int arow = wm * 16 + r;
-    const int sw = apus_row_swz(r);
-    auto read_frag = [&](Frag &f, int q) {
-        const uint8_t *stg = lds + (q % NST) * STB;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint8_t *p = stg + AB + (wn * 4 + i) * 2048 + lane * 16;
+        for (int i = 0; i < TN; ++i) {
+            const uint8_t *p = stg + AB + (wn * TN + i) * B::FB + lane * 16;
             const apus_v4u lo = *reinterpret_cast<const apus_v4u *>(p);
-            const apus_v4u hi = *reinterpret_cast<const apus_v4u *>(p + 1024);
-            f.b[i] = apus_v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+            if constexpr (B::FP4) {
+                f.w[i] = apus_v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, 0, 0, 0, 0};
+                f.sw[i] = sc[B::BM * 16 + (wn * TN + i) * 256 + r * 16 + 4 * qb + g];
+            } else {
+                const apus_v4u hi = *reinterpret_cast<const apus_v4u *>(p + 1024);
+                f.w[i] = apus_v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+            }
         }
-        const uint8_t *p = stg + arow * 128;
-        const apus_v4u lo = *reinterpret_cast<const apus_v4u *>(p + ((g ^ sw) << 4));
-        const apus_v4u hi = *reinterpret_cast<const apus_v4u *>(p + (((4 + g) ^ sw) << 4));
-        f.a = apus_v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-        f.sa = (int)apus_e8m0_of(lsc[q * BM + arow]);
+#pragma unroll
+        for (int t = 0; t < TM; ++t) {
+            const int ar = (wm * TM + t) * 16 + r;
+            const uint8_t *p = stg + ar * 128;
+            const apus_v4u lo = *reinterpret_cast<const apus_v4u *>(p + ((g ^ sw) << 4));
+            const apus_v4u hi = *reinterpret_cast<const apus_v4u *>(p + (((4 + g) ^ sw) << 4));
+            f.a[t] = apus_v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+            f.sa[t] = *reinterpret_cast<const float *>(sc + ar * 16 + 4 * qb);
+        }
     };
-    /* stage q is in LDS once at most (stages issued after it) x LPW loads
-     * are in flight: NST - 1 stages follow stage 0 before the loop; in the
-     * loop stage_ready(q) runs before stage q + NST - 1 is issued */
-    auto stage_ready = [&](int q) {
-        const int last = q == 0 ? NST - 1 : (q + NST - 2 < NQ - 1 ? q + NST - 2 : NQ - 1);
-        const int ahead = last - q;
-        if (ahead >= 3) apus_wait_vm<3 * LPW>();
-        else if (ahead == 2) apus_wait_vm<2 * LPW>();
-        else if (ahead == 1) apus_wait_vm<LPW>();
-        else apus_wait_vm<0>();
-        apus_lds_barrier();
+    apus_v4f part[B::FOLD ? TN : 1][B::FOLD ? TM : 1];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int t = 0; t < TM; ++t) {
+            acc[i][t] = apus_v4f{0.f, 0.f, 0.f, 0.f};
+            if constexpr (B::FOLD) part[i][t] = apus_v4f{0.f, 0.f, 0.f, 0.f};
+        }
+    auto mul = [&](const Frag &f, int q) {
+        const int s8 = B::FP4 ? 0 : sbw(q);
+        int sa[TM];
+#pragma unroll
+        for (int t = 0; t < TM; ++t) sa[t] = (int)apus_e8m0_of(f.sa[t]);
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int t = 0; t < TM; ++t) {
+                apus_v4f &c = [&]() -> apus_v4f & {
+                    if constexpr (B::FOLD) return part[i][t];
+                    else return acc[i][t];
+                }();
+                if constexpr (B::FP4)
+                    c = apus_mfma_scaled<APUS_FMT_E2M1, APUS_FMT_E4M3, 0, 0>(f.w[i], f.a[t], c, f.sw[i], sa[t]);
+                else
+                    c = apus_mfma_scaled<APUS_FMT_E4M3, APUS_FMT_E4M3, 0, 0>(f.w[i], f.a[t], c, s8, sa[t]);
+                /* the step's MFMAs stay in the step: moved down into the
+                 * caller's row test they would run under its lane mask, which
+                 * an MFMA does not honour and its operands' loads do */
+                if constexpr (B::NW > 4) asm volatile("" : "+v"(c));
+                else                     asm volatile("" : "+a"(c));
+            }
     };
-    static_assert(NST <= 4, "stage_ready waits for at most 3 stages ahead");
+    /* the next step's fragment reads spread among this step's MFMAs (left to
+     * itself the compiler puts them after the last, right before the wait) */
+    auto weave = [&]() {
+        constexpr int NR = 2 * TM + (B::FP4 ? 2 : 2) * TN + TM, NM = TM * TN;
+#pragma unroll
+        for (int i = 0; i < NM; ++i) {
+            constexpr int PER = (NR + NM - 1) / NM;
+            __builtin_amdgcn_sched_group_barrier(0x100, PER, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+    };
+    auto fold = [&]() {
+        if constexpr (B::FOLD) {
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+#pragma unroll
+                for (int t = 0; t < TM; ++t) {
+                    acc[i][t] += part[i][t];
+                    part[i][t] = apus_v4f{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    };
+#pragma unroll
+    for (int q = 0; q < NST; ++q) issue(q, q, q % 4 == 0);
     Frag fr[2];
-    stage_ready(0);
-    read_frag(fr[0], 0);
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        if (q + 1 < NQ) {
-            stage_ready(q + 1);
-            if (q + NST < NQ) issue(q + NST, (q + NST) % NST);
-            read_frag(fr[(q + 1) & 1], q + 1);
-        }
-        const Frag &f = fr[q & 1];
-        const int sbq = (int)((sbw[q >> 2] >> (8 * (q & 3))) & 0xffu);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            acc[i] = apus_mfma_scaled<APUS_FMT_E4M3, APUS_FMT_E4M3, 0, 0>(f.a, f.b[i], acc[i], f.sa, sbq);
+    apus_wait_vm<B::behind(0, NST - 1)>();
+    apus_lds_barrier();
+    read(fr[0], 0, 0, 0);
+    /* step q: stage q + 1 complete in every wave; slot q % NST (read by all
+     * before this barrier) takes stage q + NST; fragments q + 1; MFMAs q */
+    int slot = 0;                                            /* q % NST */
+#pragma unroll 1
+    for (int q0 = 0; q0 + 4 < NQ; q0 += 4) {
+        auto step = [&](auto jc) {
+            constexpr int j = jc;
+            const int q = q0 + j, nxt = slot + 1 == NST ? 0 : slot + 1;
+            apus_wait_vm<B::behind(j + 1, j + NST - 1)>();
+            apus_lds_barrier();
+            issue(q + NST, slot, (j + NST) % 4 == 0);
+            __builtin_amdgcn_sched_barrier(0);
+            read(fr[(j + 1) & 1], q + 1, nxt, (j + 1) & 3);
+            mul(fr[j & 1], q);
+            weave();
+            __builtin_amdgcn_sched_barrier(0);
+            if (B::FOLD && (q + 1) % (NQ / 4) == 0) fold();
+            slot = nxt;
+        };
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
     }
-    /* lane holds D[4g + j][r]: token m0 + 16 wm + 4 g + j, weight row n0 + 64 wn + 16 i + r */
+    auto tail = [&](auto jc) {
+        constexpr int j = jc, q = NQ - 4 + j;
+        const int nxt = slot + 1 == NST ? 0 : slot + 1;
+        if constexpr (q + 1 < NQ) {
+            constexpr int last = q + NST - 1 < NQ - 1 ? q + NST - 1 : NQ - 1;
+            apus_wait_vm<B::behind(q + 1, last)>();
+            apus_lds_barrier();
+            if constexpr (q + NST < NQ) issue(q + NST, slot, (q + NST) % 4 == 0);
+            __builtin_amdgcn_sched_barrier(0);
+            read(fr[(j + 1) & 1], q + 1, nxt, (j + 1) & 3);
+        }
+        mul(fr[j & 1], q);
+        if constexpr (q + 1 < NQ) weave();
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (B::FOLD && (q + 1) % (NQ / 4) == 0) fold();
+        slot = nxt;
+    };
+    tail(std::integral_constant<int, 0>{});
+    tail(std::integral_constant<int, 1>{});
+    tail(std::integral_constant<int, 2>{});
+    tail(std::integral_constant<int, 3>{});
+}
+
+/* the NQ tile scale bytes at p, byte q in lane q: scalar loads, so that none is
+ * counted among the loop's vector loads */
+template <int NQ>
+__device__ __forceinline__ int apus_block_tile_scales(const uint8_t *p) {
+    const int lane = threadIdx.x & 63;
+    unsigned v = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int mm = m0 + wm * 16 + 4 * g + j;
+    for (int i = 0; i < NQ / 4; ++i) {
+        const unsigned w = __builtin_amdgcn_readfirstlane(apus_gld<unsigned>(p + 4 * i));
+        v = (lane >> 2) == i ? w : v;
+    }
+    return (int)((v >> (8 * (lane & 3))) & 0xffu);
+}
+
+/* tile of workgroup b: each XCD (workgroups are dealt to the 8 XCDs round
+ * robin) takes a contiguous band of tiles, ordered in groups of up to 8 row
+ * blocks by every column block, so that the tiles running together on an XCD
+ * share both operands in its L2 */
+__device__ __forceinline__ void apus_block_tile(int b, int mt, int nt, int &mb, int &nb) {
+    const int tiles = mt * nt, per = tiles >> 3, rem = tiles & 7, x = b & 7;
+    const int t = x * per + min(x, rem) + (b >> 3);
+    const int grp = t / (8 * nt), g0 = grp * 8, gm = min(8, mt - g0), in = t - grp * 8 * nt;
+    mb = g0 + in % gm;
+    nb = in / gm;
+}
+
+/* dense GEMM on the block schedule: FP8 or MXFP4 tiled weights, one entry,
+ * plain row ranges, O % BN == 0 */
+template <int WF, int NQ, int BM, int BN, int WM, int WN, int NST>
+__global__ __launch_bounds__(64 * WM * WN) void apus_gemm_block_kernel(ApusGemmArgs args) {
+    typedef ApusBlk<WF, NQ, BM, BN, WM, WN, NST> B;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const ApusGemmEnt ent = args.ent0;
+    const int M = ent.M, mt = (M + BM - 1) / BM, nt = args.O / BN;
+    int mb, nb;
+    apus_block_tile(blockIdx.x, mt, nt, mb, nb);
+    const int m0 = mb * BM, n0 = nb * BN;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
+    /* FP8: 128 x 128 tile scales of the wave's columns */
+    static_assert(BN / WN <= 128, "one tile scale per wave");
+    const uint8_t *wsp = ent.ws + (size_t)((n0 + wn * (BN / WN)) >> 7) * NQ;
+    const int sb = WF == APUS_W_FP8 ? apus_block_tile_scales<NQ>(wsp) : 0;
+    apus_v4f acc[B::TN][B::TM];
+    apus_block_loop<B>(
+        lds, args.acodes + (size_t)(ent.a0 + m0) * B::K, args.ascale + (size_t)(ent.a0 + m0) * NQ,
+        [&](int i) { return min(i, M - 1 - m0); },
+        [&](int t) { return ent.w + ((size_t)(n0 >> 4) + t) * NQ * B::FB; },
+        [&](int t) { return ent.ws + ((size_t)(n0 >> 4) + t) * (NQ / 4) * 256; },
+        [&](int q) { return __builtin_amdgcn_readlane(sb, q); }, acc);
+    /* lane: row m0 + 16 (..) + r, columns 4 g .. 4 g + 3 of each weight tile */
+#pragma unroll
+    for (int t = 0; t < B::TM; ++t) {
+        const int mm = m0 + (wm * B::TM + t) * 16 + r;
         if (mm < M) {
-            float *d = ent.out + (size_t)(ent.o0 + mm) * args.ldo + n0 + wn * 64 + r;
+            float *d = ent.out + (size_t)(ent.o0 + mm) * args.ldo + n0 + wn * (BN / WN) + 4 * g;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float v = acc[i][j];
-                if (args.round_out) v = apus_bf16_rne(v);
-                apus_gst<float>(d + i * 16, v);
+            for (int i = 0; i < B::TN; ++i) {
+                apus_v4f v = acc[i][t];
+                if (args.round_out) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[j] = apus_bf16_rne(v[j]);
+                }
+                apus_gst<apus_v4f>(d + 16 * i, v);
             }
         }
     }
+}
+
+template <int WF, int NQ, int BM, int BN, int WM, int WN, int NST>
+bool apus_launch_block_tile(const ApusGemmArgs &a, hipStream_t st) {
+    typedef ApusBlk<WF, NQ, BM, BN, WM, WN, NST> B;
+    static const hipError_t attr = hipFuncSetAttribute(
+        reinterpret_cast<const void *>(&apus_gemm_block_kernel<WF, NQ, BM, BN, WM, WN, NST>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, B::LDS);
+    if (attr != hipSuccess) return false;
+    const size_t tiles = (size_t)((a.ent0.M + BM - 1) / BM) * (a.O / BN);
+    hipLaunchKernelGGL((apus_gemm_block_kernel<WF, NQ, BM, BN, WM, WN, NST>), dim3((unsigned)tiles), dim3(64 * WM * WN),
+                       B::LDS, st, a);
+    return true;
+}
+
+/* The tile: the largest that still gives most of the 256 CUs a workgroup and
+ * pads few rows. A larger tile needs fewer LDS and L2 bytes per MFMA (what
+ * bounds the loop), but a workgroup's time does not shrink when CUs idle.
+ * Measured with the act quant, us, [rows, O, K] FP8 unless said (tiles
+ * 256 x 128 / 128 x 128 / 64 x 128 / 64 x 64; workgroups of the first / last;
+ * before):
+ *   1000 x 32768 x 1024    74.6 / 93.2 / 81.3 / 89.5   1024 /        121.6
+ *   1000 x 4096 x 8192     65.0 / 48.3 / 53.9 / 66.1    128 /         60.3
+ *   512 x 4096 x 4096      34.7 / 22.7 / 18.4 / 20.4                  19.1
+ *   300 x 32768 x 1024     31.8 / 27.6 / 24.3 / 26.5   512 (70 % padding) 28.1
+ *   1000 x 1024 x 4096     36.6 / 24.3 / 18.1 / 15.9        / 256     18.8
+ *   100 x 4096 x 4096      29.1 / 19.6 / 14.8 / 11.9        / 128     15.4
+ *   4096 x 4096 x 8192    177.6 / 213.7 / 242.9 / 293.0               254.1
+ *   MXFP4 512 x 4096 x 4096  31.8 / 20.1 / 15.2 / 17.4                19.3
+ * 64 x 128 runs four stages deep where every CU has one workgroup, three
+ * (two workgroups a CU) past that: 18.4 / 18.9 at 256 workgroups, 27.2 / 24.3
+ * at 1280. */
+template <int WF, int NQ>
+bool apus_launch_block(const ApusGemmArgs &a, hipStream_t st) {
+    const int M = a.ent0.M;
+    auto tiles = [&](int bm, int bn) { return (size_t)((M + bm - 1) / bm) * (a.O / bn); };
+    auto fits = [&](int bm, int bn) {
+        const size_t padded = (size_t)((M + bm - 1) / bm) * bm;
+        return tiles(bm, bn) >= 224 && padded * 6 <= (size_t)M * 7;
+    };
+    if (fits(256, 128)) return apus_launch_block_tile<WF, NQ, 256, 128, 4, 2, 3>(a, st);
+    if (fits(128, 128)) return apus_launch_block_tile<WF, NQ, 128, 128, 2, 4, 4>(a, st);
+    const size_t t = tiles(64, 128);
+    if (t > 256) return apus_launch_block_tile<WF, NQ, 64, 128, 2, 2, 3>(a, st);
+    if (t >= 224) return apus_launch_block_tile<WF, NQ, 64, 128, 2, 2, 4>(a, st);
+    return apus_launch_block_tile<WF, NQ, 64, 64, 2, 2, 4>(a, st);
 }
 
 /*
@@ -1995,25 +2194,12 @@ void apus_launch_grp(const ApusGemmArgs &a, int n_ent, hipStream_t st) {
 }
 
 /* launch the LDS tile schedule (returns false where it does not apply) */
-template <int NQ>
-bool apus_launch_lds_tile(const ApusGemmArgs &a, hipStream_t st) {
-    constexpr int NST = APUS_LT_NST < NQ ? APUS_LT_NST : NQ;
-    constexpr size_t lds = (size_t)NST * (64 + 128) * 128 + 64 * NQ * 4;
-    static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void *>(&apus_gemm_lds_kernel<NQ>), hipFuncAttributeMaxDynamicSharedMemorySize,
-        (int)lds);
-    if (attr != hipSuccess) return false;
-    const int tiles = (a.ent0.M + 63) / 64 * (a.O / 128);
-    hipLaunchKernelGGL(apus_gemm_lds_kernel<NQ>, dim3(tiles), dim3(512), lds, st, a);
-    return true;
-}
-
 /*
  * LDS many-row schedule for the routed MXFP4 experts (grouped launches from
  * the route kernel's work list, MFMA-tiled weights, K 2048 / 4096): one
  * workgroup per (64-row chunk of an expert, 128 weight rows), whole K, both
  * operands global -> LDS through NST stages of one 128-group as in
- * apus_gemm_lds_kernel: per stage 8 loads of 8 gathered activation rows
+ * apus_block_loop: per stage 8 loads of 8 gathered activation rows
  * (row table of the entry) and 8 loads of 1 KB weight fragments (FP4: a
  * 16-row tile's 128-group is 1 KB); the weight scales of the 8 tiles (one
  * contiguous block) and the chunk's activation scales go to LDS up front.
@@ -3228,8 +3414,8 @@ bool apus_split_on() {
     return on;
 }
 
-/* the LDS tile schedule for dense FP8 GEMMs (APUS_HIP_LDS_TILE=0 turns it
- * off: the register-ring tile schedule, identical bits) */
+/* the block schedule for dense GEMMs on tiled weights (APUS_HIP_LDS_TILE=0
+ * turns it off: the register-ring tile schedule, identical bits) */
 bool apus_lds_tile_on() {
     static const bool on = [] {
         const char *e = getenv("APUS_HIP_LDS_TILE");
@@ -3449,15 +3635,20 @@ hipError_t apus_launch_gemm(int wfmt, const ApusGemmArgs *a, int n_ent,
             }
             if (ok) return hipGetLastError();
         }
-        /* FP8 on tiled weights, plain row ranges: the LDS tile schedule */
-        if (wfmt == APUS_W_FP8 && a->wtiled && !a->ent0.arows && !a->ent0.orows && apus_lds_tile_on()) {
+        /* tiled weights, plain row ranges, outputs and scales that 16-byte
+         * accesses can take: the block schedule */
+        if (a->wtiled && !a->ent0.arows && !a->ent0.orows && a->ldo % 4 == 0 &&
+            ((reinterpret_cast<uintptr_t>(a->ent0.out) | reinterpret_cast<uintptr_t>(a->ascale)) & 15) == 0 &&
+            apus_lds_tile_on()) {
             bool ok = false;
+#define APUS_BLOCK(NQ) ok = wfmt == APUS_W_FP4 ? apus_launch_block<APUS_W_FP4, NQ>(*a, st) : apus_launch_block<APUS_W_FP8, NQ>(*a, st)
             switch (a->K) {
-            case 1024: ok = apus_launch_lds_tile<8>(*a, st); break;
-            case 2048: ok = apus_launch_lds_tile<16>(*a, st); break;
-            case 4096: ok = apus_launch_lds_tile<32>(*a, st); break;
-            default:   ok = apus_launch_lds_tile<64>(*a, st); break;
+            case 1024: APUS_BLOCK(8); break;
+            case 2048: APUS_BLOCK(16); break;
+            case 4096: APUS_BLOCK(32); break;
+            default:   APUS_BLOCK(64); break;
             }
+#undef APUS_BLOCK
             if (ok) return hipGetLastError();
         }
         if (wfmt == APUS_W_FP4) {

@@ -49,3 +49,52 @@ def test_narrow_tiled(hip, oracle, rng, M, K):
     w, ws = fp8_weights(rng, O, K)
     c, s = oracle.act_quant(acts(rng, M, K, 2.0))
     check(gemm_tiled(hip, 1, w, ws, c, s), oracle, 1, w, ws, c, s)
+
+
+def gemm_rows(hip, fmt, w, ws, c, s, round_out=0):
+    """the same GEMM on row-major weights (the register-ring tile schedule)"""
+    L = hip.lib()
+    (M, K), O = c.shape, w.shape[0]
+    bufs = [hip.DevBuf.from_array(v) for v in (w, ws, c, s)]
+    do = hip.DevBuf(M * O * 4)
+    fn = L.apus_hip_fp4_gemm_dev if fmt == 0 else L.apus_hip_fp8_gemm_dev
+    hip._check(fn(*(b.ptr for b in bufs), do.ptr, M, O, K, round_out), "gemm")
+    hip._check(L.apus_hip_synchronize(), "sync")
+    return do.to_array(np.float32, (M, O))
+
+
+@pytest.mark.parametrize("fmt,M,O,K", [
+    (1, 500, 14336, 1024), (0, 449, 14336, 1024),      # 256 x 128 tiles
+    (1, 120, 28672, 1024), (0, 380, 10240, 2048),      # 128 x 128
+    (1, 65, 16384, 1024), (1, 200, 8192, 2048),        # 64 x 128, 256 workgroups; more
+    (1, 66, 128, 8192), (0, 9, 128, 1024), (1, 129, 384, 4096), (0, 64, 256, 4096), (0, 70, 128, 2048),  # 64 x 64
+    (1, 1000, 1024, 4096),
+])
+def test_block_schedule(hip, oracle, rng, fmt, M, O, K):
+    """Every tile of the block schedule, at ragged row counts: the bits of the
+    register-ring tile schedule (one chain per output in both), and the
+    oracle's values in sampled rows and columns."""
+    w, ws = (fp4_weights if fmt == 0 else fp8_weights)(rng, O, K)
+    c, s = oracle.act_quant(acts(rng, M, K, 2.0))
+    got = gemm_tiled(hip, fmt, w, ws, c, s)
+    assert np.array_equal(got.view(np.uint32), gemm_rows(hip, fmt, w, ws, c, s).view(np.uint32))
+    rows = np.unique(np.r_[0, M - 1, rng.integers(0, M, 6)])
+    cols = slice(O - 128, O)
+    wsc = ws[cols] if fmt == 0 else ws[-1:]
+    check(got[rows, cols], oracle, fmt, np.ascontiguousarray(w[cols]), np.ascontiguousarray(wsc), c[rows], s[rows])
+
+
+def test_block_schedule_unaligned_out(hip, oracle, rng):
+    """Output rows that 16-byte stores cannot take: the tile schedule, same bits."""
+    M, O, K = 70, 128, 1024
+    L = hip.lib()
+    w, ws = fp8_weights(rng, O, K)
+    c, s = oracle.act_quant(acts(rng, M, K))
+    _, _, (tw, _) = dev_pack(hip, 1, w, ws, O, K)
+    dws, dc, ds = (hip.DevBuf.from_array(v) for v in (ws, c, s))
+    do = hip.DevBuf(M * O * 4 + 16)
+    hip._check(L.apus_hip_fp8_gemm_dev(tw.ptr, dws.ptr, dc.ptr, ds.ptr, do.ptr + 4, M, O, K, hip.W_TILED | 1), "gemm")
+    hip._check(L.apus_hip_synchronize(), "sync")
+    got = do.to_array(np.float32, (M * O + 4,))[1:1 + M * O].reshape(M, O)
+    want = gemm_tiled(hip, 1, w, ws, c, s, 1)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
