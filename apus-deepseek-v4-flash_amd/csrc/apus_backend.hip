@@ -781,9 +781,25 @@ int moe_pipeline(int E, int dim, int inter, float limit, uint8_t *const *tab,
         d.O = 2 * inter; d.K = dim; d.ldo = 2 * inter; d.round_out = 1;
         if (!launched(apus_launch_gemm(APUS_W_FP8, &d, 1, st), "dense rider")) return 1;
     }
+    /* the many-row entries run from the route kernel's work list (balanced
+     * row chunks) where the many-row schedules apply */
+    const bool use_items = (dim == 2048 || dim == 4096) && (inter == 2048 || inter == 4096);
+    /* MXFP4 tiled experts, sixteen or more pairs an expert on average: the
+     * many-row items' w1/w3 on the block schedule, which hands w2 quantised h
+     * (its 32-bit row offsets reach 4 GiB), and eo stored as the BF16 values it
+     * holds where the schedules of w2 can (inter 2048; 16-byte rows of y).
+     * us without / with it, 256 experts, top-6: 4096 tokens 1440 / 1226, 2048
+     * 900 / 848, 1024 723 / 697; 512 605-611 / 603-609, 130 x top-8 540 / 548:
+     * with fewer rows an expert the weights bound both, and the few-row
+     * experts' h costs a launch over their table */
+    const bool block = use_items && wtiled && inter == 2048 && apus_moe_block_on() && (size_t)s * dim < (1ull << 32) &&
+                       w.n_items < 32768 && nj >= 16 * E &&
+                       ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(add_src) |
+                         reinterpret_cast<uintptr_t>(add_out)) & 15) == 0;
+    const int n_items128 = block ? apus_moe_items_bound(nj, E, SMALL, 128) : 0;
     if (!launched(apus_launch_moe_route(idx, nj, topk, E, t, w.gm, w.um, w.eo, w.pair, w.tok,
                                         w.e13s, w.e2s, w.e13l, w.e2l, SMALL, w.items13, w.items2,
-                                        w.n_items, st), "moe_route"))
+                                        w.n_items, n_items128, st), "moe_route"))
         return 1;
     const int n_small = std::min(E, nj), n_large = std::min(E, nj / (SMALL + 1));
     ApusGemmArgs a{};
@@ -794,10 +810,7 @@ int moe_pipeline(int E, int dim, int inter, float limit, uint8_t *const *tab,
     b.wtiled = wtiled;
     b.acodes = w.hc; b.ascale = w.hs;
     b.O = dim; b.K = inter; b.ldo = dim; b.round_out = 1;
-    /* the many-row entries run from the route kernel's work list (one
-     * APUS_PREFILL_ROWS-row chunk per launch row, balanced) where the
-     * many-row schedule applies */
-    const bool use_items = (dim == 2048 || dim == 4096) && (inter == 2048 || inter == 4096);
+    b.out_bf16 = block;
     /* at these shapes the grouped GEMMs keep the accumulation orders of the
      * one-token kernels (w1/w3: one chain over K; w2: four K-quarter chains
      * added in order), so every token's y is bit-identical to dispatching it
@@ -812,9 +825,16 @@ int moe_pipeline(int E, int dim, int inter, float limit, uint8_t *const *tab,
         a.min_m = pass ? SMALL : 0;
         a.items = pass && use_items ? w.items13 : nullptr;
         const int rows = pass && use_items ? 2 * w.n_items : 2 * n;
+        if (pass && block) {
+            if (!launched(apus_launch_moe_w13_block(w.xc, w.xs, w.e13l, w.items13, n_items128, dim, inter, limit, w.hc,
+                                                    w.hs, st), "block w1/w3"))
+                return 1;
+            continue;
+        }
         if (!launched(apus_launch_gemm(APUS_W_FP4, &a, rows, st), "gemm w1/w3")) return 1;
     }
-    if (!launched(apus_launch_swiglu_quant(w.gm, w.um, nj, inter, limit, w.hc, w.hs, st),
+    if (!launched(block ? apus_launch_swiglu_quant_ents(w.e13s, n_small, w.gm, w.um, inter, limit, w.hc, w.hs, st)
+                        : apus_launch_swiglu_quant(w.gm, w.um, nj, inter, limit, w.hc, w.hs, st),
                   "swiglu_quant"))
         return 1;
     for (int pass = 0; pass < 2; ++pass) {
@@ -828,8 +848,10 @@ int moe_pipeline(int E, int dim, int inter, float limit, uint8_t *const *tab,
         if (!launched(apus_launch_gemm(APUS_W_FP4, &b, rows, st), "gemm w2")) return 1;
     }
     if (add_out && !wait_add()) return 1;
-    if (!launched(apus_launch_moe_accum(w.eo, wgt, s, topk, dim, y, add_out ? add_src : nullptr,
-                                        add_out, st), "moe_accum"))
+    if (!launched(block ? apus_launch_moe_accum_bf16(reinterpret_cast<const uint16_t *>(w.eo), wgt, s, topk, dim, y,
+                                                     add_out ? add_src : nullptr, add_out, st)
+                        : apus_launch_moe_accum(w.eo, wgt, s, topk, dim, y, add_out ? add_src : nullptr, add_out, st),
+                  "moe_accum"))
         return 1;
     return 0;
 }

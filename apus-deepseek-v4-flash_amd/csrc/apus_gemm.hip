@@ -686,6 +686,9 @@ __attribute__((amdgpu_waves_per_eu(FOLD && NS == 4 ? APUS_DEC_FOLD_WPE : 1))) vo
                 float *dst = ent.out + (size_t)orow * args.ldo + o;
                 if (args.acc_y) /* device-coherent store: read by another workgroup */
                     __hip_atomic_store(dst, val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else if (WF == APUS_W_FP4 && ASRC == APUS_A_CODES && (FOLD || KS == 4) && args.out_bf16)
+                    apus_gst<uint16_t>(reinterpret_cast<uint16_t *>(ent.out) + (size_t)orow * args.ldo + o,
+                                       apus_bf16_bits(val));
                 else
                     apus_gst<float>(dst, val);
             }
@@ -909,7 +912,7 @@ __global__ __launch_bounds__(APUS_PRE_THREADS, APUS_PRE_WAVES >= 16 ? 1 : 2) voi
 #ifndef APUS_PRE_RA_PD
 #define APUS_PRE_RA_PD 2
 #endif
-template <int NS, bool FOLD, int NCB>
+template <int NS, bool FOLD, int NCB, bool OB>
 __global__ __launch_bounds__(512, 2) void apus_gemm_prefill_ra_kernel(ApusGemmArgs args) {
     constexpr int K = NS * 512, NQ = NS * 4, TT = 4, ROWS = 64, PD = APUS_PRE_RA_PD, NW = 8;
     constexpr int KP = 2048, NPH = K / KP, SPH = KP / 512;    /* staged K per phase, phases */
@@ -999,7 +1002,9 @@ __global__ __launch_bounds__(512, 2) void apus_gemm_prefill_ra_kernel(ApusGemmAr
                 if (t * 16 + 4 * g + q < rows) {
                     float val = FOLD ? tot[FOLD ? cb : 0][t][q] : acc[cb][t][q];
                     if (args.round_out) val = apus_bf16_rne(val);
-                    apus_gst<float>(ent.out + ((size_t)orow[t][q] * args.ldo + o), val);
+                    const size_t oi = (size_t)orow[t][q] * args.ldo + o;
+                    if constexpr (OB) apus_gst<uint16_t>(reinterpret_cast<uint16_t *>(ent.out) + oi, apus_bf16_bits(val));
+                    else              apus_gst<float>(ent.out + oi, val);
                 }
             }
         }
@@ -1073,13 +1078,20 @@ __global__ __launch_bounds__(512, 2) void apus_gemm_prefill_ra_kernel(ApusGemmAr
 template <int NS, bool FOLD>
 bool apus_launch_pre_ra(const ApusGemmArgs &p, int n_ent, hipStream_t st) {
     constexpr size_t lds = 64 * (2048 + 32) + 64 * (NS * 4);
-    static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void *>(&apus_gemm_prefill_ra_kernel<NS, FOLD, APUS_PRE_RA_NCB>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (attr != hipSuccess) return false;
     dim3 gr(p.O / (128 * APUS_PRE_RA_NCB), n_ent);
-    hipLaunchKernelGGL((apus_gemm_prefill_ra_kernel<NS, FOLD, APUS_PRE_RA_NCB>), gr, dim3(512), lds, st, p);
-    return true;
+    auto go = [&](auto obc) {
+        constexpr bool OB = obc;
+        static const hipError_t attr = hipFuncSetAttribute(
+            reinterpret_cast<const void *>(&apus_gemm_prefill_ra_kernel<NS, FOLD, APUS_PRE_RA_NCB, OB>),
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (attr != hipSuccess) return false;
+        hipLaunchKernelGGL((apus_gemm_prefill_ra_kernel<NS, FOLD, APUS_PRE_RA_NCB, OB>), gr, dim3(512), lds, st, p);
+        return true;
+    };
+    if constexpr (FOLD) {
+        if (p.out_bf16) return go(std::true_type{});
+    }
+    return go(std::false_type{});
 }
 
 /*
@@ -1329,13 +1341,12 @@ __global__ __launch_bounds__(64 * NW) void apus_gemm_tile_kernel(ApusGemmArgs ar
  * loads into registers, the compiler would drain all of them at each use.
  * The weights are the MFMA's first operand, so a lane ends up with four
  * consecutive outputs of one row. Every output is one chain over the
- * 128-groups in order, as in the smaller tiles (identical bits); with FOLD,
- * four chains over the quarters of K, added in order.
+ * 128-groups in order, as in the smaller tiles (identical bits).
  */
-template <int WF, int NQ_, int BM_, int BN_, int WM_, int WN_, int NST_, bool FOLD_ = false>
+template <int WF, int NQ_, int BM_, int BN_, int WM_, int WN_, int NST_>
 struct ApusBlk {
     static constexpr int NQ = NQ_, BM = BM_, BN = BN_, WM = WM_, WN = WN_, NST = NST_, NW = WM * WN;
-    static constexpr bool FP4 = WF == APUS_W_FP4, FOLD = FOLD_;
+    static constexpr bool FP4 = WF == APUS_W_FP4;
     static constexpr int TM = BM / 16 / WM, TN = BN / 16 / WN, K = NQ * 128;
     static constexpr int FB = FP4 ? 1024 : 2048;             /* bytes of a weight fragment */
     static constexpr int AB = BM * 128, STB = AB + BN / 16 * FB;
@@ -1439,14 +1450,10 @@ __device__ __forceinline__ void apus_block_loop(uint8_t *lds, const uint8_t *aco
             f.sa[t] = *reinterpret_cast<const float *>(sc + ar * 16 + 4 * qb);
         }
     };
-    apus_v4f part[B::FOLD ? TN : 1][B::FOLD ? TM : 1];
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
-        for (int t = 0; t < TM; ++t) {
-            acc[i][t] = apus_v4f{0.f, 0.f, 0.f, 0.f};
-            if constexpr (B::FOLD) part[i][t] = apus_v4f{0.f, 0.f, 0.f, 0.f};
-        }
+        for (int t = 0; t < TM; ++t) acc[i][t] = apus_v4f{0.f, 0.f, 0.f, 0.f};
     auto mul = [&](const Frag &f, int q) {
         const int s8 = B::FP4 ? 0 : sbw(q);
         int sa[TM];
@@ -1456,10 +1463,7 @@ __device__ __forceinline__ void apus_block_loop(uint8_t *lds, const uint8_t *aco
         for (int i = 0; i < TN; ++i)
 #pragma unroll
             for (int t = 0; t < TM; ++t) {
-                apus_v4f &c = [&]() -> apus_v4f & {
-                    if constexpr (B::FOLD) return part[i][t];
-                    else return acc[i][t];
-                }();
+                apus_v4f &c = acc[i][t];
                 if constexpr (B::FP4)
                     c = apus_mfma_scaled<APUS_FMT_E2M1, APUS_FMT_E4M3, 0, 0>(f.w[i], f.a[t], c, f.sw[i], sa[t]);
                 else
@@ -1474,23 +1478,12 @@ __device__ __forceinline__ void apus_block_loop(uint8_t *lds, const uint8_t *aco
     /* the next step's fragment reads spread among this step's MFMAs (left to
      * itself the compiler puts them after the last, right before the wait) */
     auto weave = [&]() {
-        constexpr int NR = 2 * TM + (B::FP4 ? 2 : 2) * TN + TM, NM = TM * TN;
+        constexpr int NR = 3 * TM + 2 * TN, NM = TM * TN;
 #pragma unroll
         for (int i = 0; i < NM; ++i) {
             constexpr int PER = (NR + NM - 1) / NM;
             __builtin_amdgcn_sched_group_barrier(0x100, PER, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        }
-    };
-    auto fold = [&]() {
-        if constexpr (B::FOLD) {
-#pragma unroll
-            for (int i = 0; i < TN; ++i)
-#pragma unroll
-                for (int t = 0; t < TM; ++t) {
-                    acc[i][t] += part[i][t];
-                    part[i][t] = apus_v4f{0.f, 0.f, 0.f, 0.f};
-                }
         }
     };
 #pragma unroll
@@ -1515,7 +1508,6 @@ __device__ __forceinline__ void apus_block_loop(uint8_t *lds, const uint8_t *aco
             mul(fr[j & 1], q);
             weave();
             __builtin_amdgcn_sched_barrier(0);
-            if (B::FOLD && (q + 1) % (NQ / 4) == 0) fold();
             slot = nxt;
         };
         step(std::integral_constant<int, 0>{});
@@ -1537,7 +1529,6 @@ __device__ __forceinline__ void apus_block_loop(uint8_t *lds, const uint8_t *aco
         mul(fr[j & 1], q);
         if constexpr (q + 1 < NQ) weave();
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (B::FOLD && (q + 1) % (NQ / 4) == 0) fold();
         slot = nxt;
     };
     tail(std::integral_constant<int, 0>{});
@@ -1659,6 +1650,108 @@ bool apus_launch_block(const ApusGemmArgs &a, hipStream_t st) {
     if (t > 256) return apus_launch_block_tile<WF, NQ, 64, 128, 2, 2, 3>(a, st);
     if (t >= 224) return apus_launch_block_tile<WF, NQ, 64, 128, 2, 2, 4>(a, st);
     return apus_launch_block_tile<WF, NQ, 64, 64, 2, 2, 4>(a, st);
+}
+
+/*
+ * w1 and w3 of the routed experts with more than 8 rows, on the block schedule
+ * (MXFP4 tiled weights), SwiGLU and the act quant of h included. A workgroup
+ * of 8 waves takes up to 128 rows of one expert (a 128-row tile where it has
+ * more than 64 left, else a 64-row one) and 128 weight rows of w1 and the same
+ * 128 of w3, a wave holding both for its columns. So it has whole 128-column
+ * groups of g and u: it forms h = swiglu(bf16 g, bf16 u), the group maximum
+ * over its waves and the E4M3 codes of h with the steps of
+ * apus_swiglu_quant_kernel (identical codes). Before, g and u went out as fp32
+ * and were read back by that kernel (0.8 GB at 4096 tokens x top-6).
+ * 4096 tokens x top-6, 256 experts, Zipf token ids: 690 us + 90 for that
+ * kernel -> 668 (1.23 PFLOP/s of the rows asked for, 77 % of those multiplied);
+ * 512 tokens, Zipf experts, 125 + 15 -> 135 (+ 8 for the few-row experts' rows).
+ * Bound by LDS bandwidth (128 KB a step of 128 rows) and, one workgroup a CU,
+ * by its start and end; without MFMAs it runs 596 us, without staging 521.
+ * w2 on the same loop (64 rows, its four chains) ran 477 us against 450 for the
+ * resident-activation schedule at 4096 tokens, 104 against 80 at 512: not kept.
+ */
+struct ApusMoeBlkArgs {
+    const uint8_t *acodes;    /* x codes and scales */
+    const float *ascale;
+    const ApusGemmEnt *ents;  /* many-row entries: w1 and w3 of slot i at 2 i and 2 i + 1 */
+    const int2 *items;        /* (slot, first row), 128 rows each; slot < 0: nothing */
+    int O;                    /* weight rows of one matrix */
+    float limit;
+    uint8_t *hc;              /* h codes [rows, O] and scales [rows, O / 128] */
+    float *hs;
+};
+
+template <class B>
+__device__ __forceinline__ void apus_moe_w13_body(uint8_t *lds, const ApusMoeBlkArgs &a, const ApusGemmEnt &e1,
+                                                  const ApusGemmEnt &e3, int c0) {
+    constexpr int NQ = B::NQ, TM = B::TM, TN = B::TN, HN = TN / 2, WN = B::WN;
+    static_assert(B::BN == 256 && HN * 16 * WN == 128, "128 columns of both matrices");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
+    const int nb = blockIdx.x, last = e1.M - 1;
+    /* block tile t: wave t / TN, its tiles HN of w1, then HN of w3 */
+    auto tile = [&](int t, bool &is3) {
+        is3 = t % TN >= HN;
+        return nb * 8 + t / TN * HN + t % HN;
+    };
+    apus_v4f acc[TN][TM];
+    apus_block_loop<B>(
+        lds, a.acodes, a.ascale, [&](int i) { return apus_gld<int>(e1.arows + min(c0 + i, last)); },
+        [&](int t) { bool is3; const int q = tile(t, is3); return (is3 ? e3.w : e1.w) + (size_t)q * NQ * B::FB; },
+        [&](int t) { bool is3; const int q = tile(t, is3); return (is3 ? e3.ws : e1.ws) + (size_t)q * (NQ / 4) * 256; },
+        [&](int) { return 0; }, acc);
+    /* acc[i][t] (g), acc[HN + i][t] (u): row 16 (..) + r, columns 16 (wn HN + i) + 4 g + j */
+    float *red = reinterpret_cast<float *>(lds + B::LDS);    /* [WN][BM] */
+    float h[TM][HN][4];
+#pragma unroll
+    for (int t = 0; t < TM; ++t) {
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < HN; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                h[t][i][j] = apus_swiglu_h(apus_bf16_rne(acc[i][t][j]), apus_bf16_rne(acc[HN + i][t][j]), a.limit);
+                m = fmaxf(m, fabsf(h[t][i][j]));
+            }
+        m = fmaxf(m, __shfl_xor(m, 16, 64));
+        m = fmaxf(m, __shfl_xor(m, 32, 64));
+        if (g == 0) red[wn * B::BM + (wm * TM + t) * 16 + r] = m;
+    }
+    apus_lds_barrier();
+#pragma unroll
+    for (int t = 0; t < TM; ++t) {
+        const int lr = (wm * TM + t) * 16 + r;
+        float m = red[lr];
+#pragma unroll
+        for (int k = 1; k < WN; ++k) m = fmaxf(m, red[k * B::BM + lr]);
+        const uint32_t e = apus_act_scale_exp(m);
+        const float inv = apus_inv_pow2_from_exp(e);
+        if (c0 + lr <= last) {
+            const size_t row = (size_t)(e1.o0 + c0 + lr);
+            uint8_t *d = a.hc + row * a.O + nb * 128 + wn * (HN * 16) + 4 * g;
+#pragma unroll
+            for (int i = 0; i < HN; ++i)
+                apus_gst<uint32_t>(d + 16 * i, apus_e4m3_pack4_hw(h[t][i][0] * inv, h[t][i][1] * inv,
+                                                                  h[t][i][2] * inv, h[t][i][3] * inv));
+            if (wn == 0 && g == 0) apus_gst<float>(a.hs + row * (a.O >> 7) + nb, apus_pow2_from_exp(e));
+        }
+    }
+}
+
+template <int NQ>
+struct ApusMoeW13 {
+    typedef ApusBlk<APUS_W_FP4, NQ, 128, 256, 2, 4, 3> Big;
+    typedef ApusBlk<APUS_W_FP4, NQ, 64, 256, 2, 4, 4> Small;
+    static constexpr int LDS = (Big::LDS > Small::LDS ? Big::LDS : Small::LDS) + 4 * 128 * 4;
+};
+template <int NQ>
+__global__ __launch_bounds__(512) void apus_moe_w13_block_kernel(ApusMoeBlkArgs a) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int2 it = a.items[blockIdx.y];
+    if (it.x < 0) return;
+    const ApusGemmEnt e1 = a.ents[2 * it.x], e3 = a.ents[2 * it.x + 1];
+    if (e1.M - it.y > 64) apus_moe_w13_body<typename ApusMoeW13<NQ>::Big>(lds, a, e1, e3, it.y);
+    else                  apus_moe_w13_body<typename ApusMoeW13<NQ>::Small>(lds, a, e1, e3, it.y);
 }
 
 /*
@@ -3514,6 +3607,26 @@ hipError_t apus_launch_gemm_few(int wfmt, const ApusGemmArgs *a, int n_ent, int 
         return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+bool apus_moe_block_on() { return apus_pre_lds_mode() == 1; }
+
+hipError_t apus_launch_moe_w13_block(const uint8_t *acodes, const float *ascale, const ApusGemmEnt *ents,
+                                     const int2 *items, int n_items, int K, int O, float limit, uint8_t *hc, float *hs,
+                                     hipStream_t st) {
+    if (n_items <= 0) return hipSuccess;
+    if (!apus_group_k(K) || O % 128 || (reinterpret_cast<uintptr_t>(ascale) & 15)) return hipErrorInvalidValue;
+    const ApusMoeBlkArgs a{acodes, ascale, ents, items, O, limit, hc, hs};
+    auto go = [&](auto nqc) {
+        constexpr int NQ = nqc;
+        static const hipError_t attr = hipFuncSetAttribute(
+            reinterpret_cast<const void *>(&apus_moe_w13_block_kernel<NQ>),
+            hipFuncAttributeMaxDynamicSharedMemorySize, ApusMoeW13<NQ>::LDS);
+        if (attr != hipSuccess) return attr;
+        hipLaunchKernelGGL((apus_moe_w13_block_kernel<NQ>), dim3(O / 128, n_items), dim3(512), ApusMoeW13<NQ>::LDS, st, a);
+        return hipGetLastError();
+    };
+    return K == 4096 ? go(std::integral_constant<int, 32>{}) : go(std::integral_constant<int, 16>{});
 }
 
 hipError_t apus_launch_gemm(int wfmt, const ApusGemmArgs *a, int n_ent,

@@ -50,7 +50,8 @@ typedef struct {
                               * The routed MoE uses 1 for w1/w3 and 4 for w2, the
                               * orders of its one-token kernels, so a token's
                               * result does not depend on the batch around it. */
-    int pad3;
+    int out_bf16;            /* kchain 4 on the few-row and resident-activation schedules:
+                              * outputs stored as BF16 (2 bytes each; round_out set) */
     /* --- few-row schedule only (apus_launch_gemm_few) --- */
     int asrc;                /* APUS_A_*: where the activation rows come from */
     const float *ax, *au;    /* F32: rows of x [*, K]; SWIGLU: rows of g and u [*, K] */
@@ -194,6 +195,23 @@ hipError_t apus_launch_swiglu_quant(const float *g, const float *u, int M,
                                     int N, float limit, uint8_t *codes,
                                     float *scales, hipStream_t st);
 
+/* The same over the rows of small entries (at most 8 rows each): entry
+ * ents[2 i] gives rows [o0, o0 + M) of g, u, codes and scales. */
+hipError_t apus_launch_swiglu_quant_ents(const ApusGemmEnt *ents, int n_ent, const float *g, const float *u, int N,
+                                         float limit, uint8_t *codes, float *scales, hipStream_t st);
+
+/* w1/w3 of the routed experts' many-row work items on the block schedule
+ * (MXFP4 tiled weights, K 2048 or 4096, O % 128 == 0, x rows * K below 4 GiB),
+ * with SwiGLU and act quant: h codes hc [*, O], scales hs [*, O / 128]. items:
+ * (entry slot, first row), 128 rows each. */
+hipError_t apus_launch_moe_w13_block(const uint8_t *acodes, const float *ascale, const ApusGemmEnt *ents,
+                                     const int2 *items, int n_items, int K, int O, float limit, uint8_t *hc, float *hs,
+                                     hipStream_t st);
+/* whether the routed dispatch uses it (APUS_HIP_PRE_LDS=0 turns it off: the
+ * resident-activation and prefill schedules on fp32 g, u and eo, identical
+ * results) */
+bool apus_moe_block_on();
+
 /* Counting sort of the routed pairs by expert and GEMM entry tables.
  * idx [nj] (nj = s * topk) expert ids in [0, E), E <= 1024; writes
  * pair_sorted [nj] (pair q), tok_sorted [nj] (q / topk) and two sets of
@@ -202,7 +220,9 @@ hipError_t apus_launch_swiglu_quant(const float *g, const float *u, int M,
  * order) and e2s [E] (output rows = pair ids); experts with more pairs go to
  * e13l / e2l the same way. Slots past the listed experts have M = 0.
  * items13 [2 n_items] / items2 [n_items] list (entry, first row) of every
- * APUS_PREFILL_ROWS-row chunk of the many-row entries (x = -1 past the end).
+ * APUS_PREFILL_ROWS-row chunk of the many-row entries (x = -1 past the end);
+ * with n_items128 > 0, items13 [n_items128] instead lists (slot, first row) of
+ * every 128-row chunk (n_items < 32768).
  * The weight pointer tables are device arrays of E pointers each. */
 typedef struct {
     const uint8_t *const *w1, *const *w1s, *const *w2, *const *w2s,
@@ -214,12 +234,12 @@ hipError_t apus_launch_moe_route(const int32_t *idx, int nj, int topk, int E,
                                  int32_t *pair_sorted, int32_t *tok_sorted,
                                  ApusGemmEnt *e13s, ApusGemmEnt *e2s, ApusGemmEnt *e13l,
                                  ApusGemmEnt *e2l, int small_max, int2 *items13, int2 *items2,
-                                 int n_items, hipStream_t st);
+                                 int n_items, int n_items128, hipStream_t st);
 
 /* work-list bound per matrix for the many-row experts of nj pairs */
-static inline int apus_moe_items_bound(int nj, int E, int small_max) {
+static inline int apus_moe_items_bound(int nj, int E, int small_max, int rows = APUS_PREFILL_ROWS) {
     const int nl = (nj / (small_max + 1)) < E ? nj / (small_max + 1) : E;
-    return nj / APUS_PREFILL_ROWS + nl;
+    return nj / rows + nl;
 }
 
 /* Row-major <-> MFMA-tiled weights (unpack = 0: w, ws -> tw, tws). FP4
@@ -252,6 +272,10 @@ hipError_t apus_launch_add_bf16(const float *a, const float *b, float *out, size
 hipError_t apus_launch_moe_accum(const float *eo, const float *wgt, int s,
                                  int topk, int dim, float *y, const float *add_src,
                                  float *add_out, hipStream_t st);
+
+/* The same from BF16 eo (dim % 8 == 0, 16-byte rows). */
+hipError_t apus_launch_moe_accum_bf16(const uint16_t *eo, const float *wgt, int s, int topk, int dim, float *y,
+                                      const float *add_src, float *add_out, hipStream_t st);
 
 /* Counter-based fill (kind as orc_fill_bytes: 0 uniform byte, 1 E8M0
  * 118..130, 2 E4M3 of ~N(0,1), 3 E8M0 117..123). */

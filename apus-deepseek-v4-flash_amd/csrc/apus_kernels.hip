@@ -125,6 +125,48 @@ hipError_t apus_launch_swiglu_quant(const float *g, const float *u, int M,
     return hipGetLastError();
 }
 
+/* The same over the rows of small entries (their w1/w3 went through the
+ * few-row schedule; the many-row entries' h comes out of their kernel already
+ * quantised): one workgroup per (128-column group, entry), 32 lanes per row
+ * (M <= 8; two workgroups an entry looping over its rows and groups instead
+ * ran 7 us longer on an entry of 8 rows). */
+__global__ __launch_bounds__(256) void apus_swiglu_quant_ents_kernel(
+    const ApusGemmEnt *__restrict__ ents, const float *__restrict__ gm, const float *__restrict__ um, int N,
+    float limit, uint8_t *__restrict__ codes, float *__restrict__ scales) {
+    const ApusGemmEnt *ent = ents + 2 * blockIdx.y;
+    const int M = ent->M, o0 = ent->o0, b = blockIdx.x;
+    const int l32 = threadIdx.x & 31, row = threadIdx.x >> 5;
+    if (M <= 0) return;
+    /* both halves of a wave take part in the shuffles: a row past the entry
+     * computes on its last one and stores nothing */
+    const int m = o0 + min(row, M - 1);
+    const size_t off = (size_t)m * N + b * 128 + l32 * 4;
+    const float4 gv = *reinterpret_cast<const float4 *>(gm + off);
+    const float4 uv = *reinterpret_cast<const float4 *>(um + off);
+    const float h[4] = {apus_swiglu_h(gv.x, uv.x, limit), apus_swiglu_h(gv.y, uv.y, limit),
+                        apus_swiglu_h(gv.z, uv.z, limit), apus_swiglu_h(gv.w, uv.w, limit)};
+    float amax = fmaxf(fmaxf(fabsf(h[0]), fabsf(h[1])), fmaxf(fabsf(h[2]), fabsf(h[3])));
+#pragma unroll
+    for (int o = 16; o >= 1; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    const uint32_t ex = apus_act_scale_exp(amax);
+    const float inv = apus_inv_pow2_from_exp(ex);
+    if (row >= M) return;
+    *reinterpret_cast<uint32_t *>(codes + off) =
+        apus_e4m3_pack4_hw(h[0] * inv, h[1] * inv, h[2] * inv, h[3] * inv);
+    if (l32 == 0) scales[(size_t)m * (N >> 7) + b] = apus_pow2_from_exp(ex);
+}
+
+hipError_t apus_launch_swiglu_quant_ents(const ApusGemmEnt *ents, int n_ent, const float *g, const float *u, int N,
+                                         float limit, uint8_t *codes, float *scales, hipStream_t st) {
+    if (n_ent <= 0) return hipSuccess;
+    if (N <= 0 || N % 128 || ((reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(u)) & 15) ||
+        (reinterpret_cast<uintptr_t>(codes) & 3))
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(apus_swiglu_quant_ents_kernel, dim3(N / 128, n_ent), dim3(256), 0, st, ents, g, u, N, limit,
+                       codes, scales);
+    return hipGetLastError();
+}
+
 /* ------------------------------------------------------------ MoE route */
 
 /* Exclusive prefix sums of three ints per thread over the workgroup (at most
@@ -171,7 +213,7 @@ __global__ __launch_bounds__(1024) void apus_moe_route_kernel(
     ApusExpertTable tab, float *g, float *u, float *eo,
     int32_t *pair_sorted, int32_t *tok_sorted, ApusGemmEnt *e13s, ApusGemmEnt *e2s,
     ApusGemmEnt *e13l, ApusGemmEnt *e2l, int small_max, int2 *items13, int2 *items2,
-    int n_items) {
+    int n_items, int n_items128) {
     __shared__ int cnt[1024], base[1024], cur[1024], sw[51];
     const int e = threadIdx.x, nt = blockDim.x;
     const bool more = nj > APUS_ROUTE_REG * nt;
@@ -205,10 +247,15 @@ __global__ __launch_bounds__(1024) void apus_moe_route_kernel(
     const int small = c > 0 && c <= small_max, large = c > small_max;
     /* work list of the many-row entries: one item per APUS_PREFILL_ROWS rows */
     const int nchunk = large ? (c + APUS_PREFILL_ROWS - 1) / APUS_PREFILL_ROWS : 0;
+    /* with n_items128, a second list of 128-row chunks, its counts in the upper
+     * halves (the launcher keeps both below 2^15) */
+    const int nchunk128 = n_items128 && large ? (c + 127) / 128 : 0;
     int3 tot;
-    const int3 sc = apus_block_scan3_excl(int3{c, small | (large << 16), nchunk}, sw, tot);
-    const int o0 = sc.x, packed = sc.y, cbase = sc.z;
-    const int ns = tot.y & 0xffff, nl = tot.y >> 16, total_chunks = tot.z;
+    const int3 sc = apus_block_scan3_excl(int3{c, small | (large << 16), nchunk | (nchunk128 << 16)}, sw, tot);
+    const int o0 = sc.x, packed = sc.y;
+    const int cbase = n_items128 ? sc.z & 0xffff : sc.z, cbase128 = sc.z >> 16;
+    const int ns = tot.y & 0xffff, nl = tot.y >> 16;
+    const int total_chunks = n_items128 ? tot.z & 0xffff : tot.z;
     base[e] = o0;
     if (more) cur[e] += o0;
     __syncthreads();
@@ -231,9 +278,11 @@ __global__ __launch_bounds__(1024) void apus_moe_route_kernel(
     if (items2) {
         for (int i = total_chunks + threadIdx.x; i < n_items; i += blockDim.x) {
             items2[i] = int2{-1, 0};
+            if (n_items128) continue;
             items13[2 * i] = int2{-1, 0};
             items13[2 * i + 1] = int2{-1, 0};
         }
+        for (int i = (tot.z >> 16) + threadIdx.x; i < n_items128; i += blockDim.x) items13[i] = int2{-1, 0};
     }
     if (e >= E) return;
     ApusGemmEnt a;
@@ -258,9 +307,12 @@ __global__ __launch_bounds__(1024) void apus_moe_route_kernel(
         for (int k = 0; k < nchunk && cbase + k < n_items; ++k) {
             const int c0 = k * APUS_PREFILL_ROWS;
             items2[cbase + k] = int2{slot, c0};
+            if (n_items128) continue;
             items13[2 * (cbase + k)] = int2{2 * slot, c0};
             items13[2 * (cbase + k) + 1] = int2{2 * slot + 1, c0};
         }
+        for (int k = 0; k < nchunk128 && cbase128 + k < n_items128; ++k)
+            items13[cbase128 + k] = int2{slot, 128 * k};
     }
 }
 
@@ -269,11 +321,12 @@ hipError_t apus_launch_moe_route(const int32_t *idx, int nj, int topk, int E,
                                  int32_t *pair_sorted, int32_t *tok_sorted,
                                  ApusGemmEnt *e13s, ApusGemmEnt *e2s, ApusGemmEnt *e13l,
                                  ApusGemmEnt *e2l, int small_max, int2 *items13, int2 *items2,
-                                 int n_items, hipStream_t st) {
-    if (E <= 0 || E > 1024) return hipErrorInvalidValue;
+                                 int n_items, int n_items128, hipStream_t st) {
+    if (E <= 0 || E > 1024 || (n_items128 && (n_items >= 32768 || n_items128 > 2 * n_items)))
+        return hipErrorInvalidValue;
     hipLaunchKernelGGL(apus_moe_route_kernel, dim3(1), dim3(1024), 0, st, idx, nj, topk, E,
                        tab, g, u, eo, pair_sorted, tok_sorted, e13s, e2s, e13l, e2l, small_max,
-                       items13, items2, n_items);
+                       items13, items2, n_items, n_items128);
     return hipGetLastError();
 }
 
@@ -521,6 +574,47 @@ hipError_t apus_launch_moe_accum(const float *eo, const float *wgt, int s,
     }
     hipLaunchKernelGGL(apus_moe_accum_kernel, dim3((dim + 255) / 256, s), dim3(256), 0, st,
                        eo, wgt, s, topk, dim, y, add_src, add_out);
+    return hipGetLastError();
+}
+
+/* The same sums from BF16 eo (the routed block schedule's: the values are
+ * BF16-rounded by contract, so half the bytes hold them), 8 columns per
+ * thread. 4096 tokens x top-6: 110 -> 81 us. */
+__global__ __launch_bounds__(256) void apus_moe_accum_bf16_kernel(
+    const uint16_t *__restrict__ eo, const float *__restrict__ wgt, int topk, int dim,
+    float *__restrict__ y, const float *__restrict__ add_src, float *__restrict__ add_out) {
+    const int i = (blockIdx.x * 256 + threadIdx.x) * 8;
+    const int t = blockIdx.y;
+    if (i >= dim) return;
+    float acc[8] = {};
+    for (int j = 0; j < topk; ++j) {
+        const float w = wgt[t * topk + j];
+        const uint4 v = *reinterpret_cast<const uint4 *>(eo + (size_t)(t * topk + j) * dim + i);
+        const uint32_t q[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            acc[2 * k] = __fadd_rn(acc[2 * k], __fmul_rn(w, __uint_as_float(q[k] << 16)));
+            acc[2 * k + 1] = __fadd_rn(acc[2 * k + 1], __fmul_rn(w, __uint_as_float(q[k] & 0xffff0000u)));
+        }
+    }
+    const size_t o = (size_t)t * dim + i;
+#pragma unroll
+    for (int k = 0; k < 8; k += 4) {
+        if (y) *reinterpret_cast<float4 *>(y + o + k) = float4{acc[k], acc[k + 1], acc[k + 2], acc[k + 3]};
+        if (add_out) {
+            const float4 a = *reinterpret_cast<const float4 *>(add_src + o + k);
+            *reinterpret_cast<float4 *>(add_out + o + k) =
+                float4{apus_bf16_rne(acc[k] + a.x), apus_bf16_rne(acc[k + 1] + a.y),
+                       apus_bf16_rne(acc[k + 2] + a.z), apus_bf16_rne(acc[k + 3] + a.w)};
+        }
+    }
+}
+
+hipError_t apus_launch_moe_accum_bf16(const uint16_t *eo, const float *wgt, int s, int topk, int dim, float *y,
+                                      const float *add_src, float *add_out, hipStream_t st) {
+    if (s <= 0) return hipSuccess;
+    hipLaunchKernelGGL(apus_moe_accum_bf16_kernel, dim3((dim / 8 + 255) / 256, s), dim3(256), 0, st, eo, wgt, topk,
+                       dim, y, add_src, add_out);
     return hipGetLastError();
 }
 

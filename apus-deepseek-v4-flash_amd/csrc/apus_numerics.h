@@ -29,6 +29,12 @@ APUS_HD float apus_bf16_rne(float x) {
     return apus_u2f(u & 0xffff0000u);
 }
 
+/* Upper half of a BF16-valued fp32 (a NaN stays a NaN). */
+APUS_HD uint16_t apus_bf16_bits(float x) {
+    const uint32_t u = apus_f2u(x);
+    return (uint16_t)((u >> 16) | ((u & 0x7fffffffu) > 0x7f800000u ? 0x40u : 0u));
+}
+
 /* fp32 -> E4M3 code (c/fp4.h:219-253): saturating clamp to +-448, then
  * round to nearest even on the E4M3 grid. For |x| >= 2^-6 the rounding is
  * done on the fp32 bits, keeping three mantissa bits (a carry walks into the

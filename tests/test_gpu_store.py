@@ -299,3 +299,45 @@ def test_routed_with_dense_rider(hip, oracle, store, rng, s):
     if s == 1:
         # rider inside the w1/w3 launch; one launch in all with the one-launch layer
         assert launches == (1 if L_.apus_hip_layer1(-1, None) == 1 else 2), launches
+
+
+@pytest.mark.parametrize("dim", [2048, 4096])
+def test_moe_routed_block_schedule(hip, oracle, store, rng, dim):
+    """Sixteen or more pairs an expert on average take the block schedule for
+    the many-row w1/w3 (128-row and 64-row tiles: experts of 129, 128, 65, 64,
+    9 and 5 rows) and BF16 expert outputs: y and the h codes equal, bit for
+    bit, those of the same tokens dispatched in batches too small for it, and
+    the first batch passes the oracle's stage checks."""
+    E, inter, s, topk, part = 8, 2048, 200, 2, 50
+    counts = [129, 128, 65, 64, 9, 5]
+    flat = rng.permutation(np.repeat(np.arange(6), counts))
+    idx = flat.reshape(s, topk).astype(np.int32)
+    assert s * topk >= 16 * E > part * topk
+    wgt = rng.random((s, topk)).astype(np.float32)
+    x = acts(rng, s, dim)
+    st = store(1, E, dim, inter)
+    L = hip.lib()
+    hip._check(L.apus_hip_store_fill_random(st, 5), "fill")
+
+    def run(a, b):
+        n = b - a
+        dx, di, dw = (hip.DevBuf.from_array(v[a:b]) for v in (x, idx, wgt))
+        dy = hip.DevBuf(n * dim * 4)
+        wsp = hip.DevBuf(L.apus_hip_moe_workspace(st, n, topk))
+        hip._check(L.apus_hip_moe_routed_dev(st, 0, dx.ptr, di.ptr, dw.ptr, n, topk, 10.0, dy.ptr, wsp.ptr),
+                   "routed")
+        hc, he = hip.DevBuf(n * topk * inter), hip.DevBuf(n * topk * inter // 128)
+        hip._check(L.apus_hip_moe_routed_h(st, n, topk, wsp.ptr, hc.ptr, he.ptr), "h")
+        return (dy.to_array(np.float32, (n, dim)), hc.to_array(np.uint8, (n * topk, inter)),
+                he.to_array(np.uint8, (n * topk, inter // 128)), wsp)
+
+    y, hc, he, _ = run(0, s)
+    for a in range(0, s, part):
+        yp, hcp, hep, wsp = run(a, a + part)
+        assert np.array_equal(y[a:a + part].view(np.uint32), yp.view(np.uint32)), a
+        assert np.array_equal(hc[topk * a:topk * (a + part)], hcp), a
+        assert np.array_equal(he[topk * a:topk * (a + part)], hep), a
+        if a == 0:
+            host = {e: host_expert(oracle, 5, 0, e, E, dim, inter) for e in range(6)}
+            stage_check(hip, oracle, st, lambda e: host[e], x[:part], idx[:part], wgt[:part], yp, wsp, inter,
+                        [0, 17, 49])
