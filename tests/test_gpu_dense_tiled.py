@@ -40,7 +40,7 @@ def check(got, oracle, fmt, w, ws, c, s):
 
 
 @pytest.mark.parametrize("K", (1024, 2048, 4096, 8192))
-@pytest.mark.parametrize("M", (9, 16, 17, 32, 33, 64))
+@pytest.mark.parametrize("M", (9, 16, 17, 32, 33, 48, 49, 64))
 def test_narrow_tiled(hip, oracle, rng, M, K):
     """The narrow schedule (FP8, 9..64 rows): tile scales that differ along K,
     at K = 1024 too, where a wave's two groups share a word of scale bytes with
