@@ -333,14 +333,30 @@ hipError_t apus_launch_moe_route(const int32_t *idx, int nj, int topk, int E,
 /* ---------------------------------------------------------------- router */
 
 /* Router scores (c/moe.h:352-367): sp[t, e] = sqrt(softplus(gate_w[e] . x[t]))
- * and, with a bias, biased = sp + bias[e] for the selection. One workgroup
- * per (expert, group of up to 8 tokens): the expert's gate row is read once
- * into registers (thread i holds float4s i, i + 256, ...), each token's dot is
- * a per-thread partial, a fixed xor-shuffle tree per wave and the four wave
- * sums in wave order. The fp32 sum order differs from the reference's
- * sequential dot (and expf/log1pf come from ROCm's libm), so scores match
- * within fp32 rounding, not bitwise. dim % 256 == 0, dim <= 8192. */
+ * and, with a bias, biased = sp + bias[e] for the selection.
+ *
+ * One order of additions for all three kernels, so a token's scores do not depend
+ * on how many tokens are scored with it: K in blocks of 16; block b is chain
+ * b % 256 (for dim > 4096 chain c takes blocks c and c + 256), a chain of fused
+ * multiply-adds over the block's elements 4 g + c in the order c = 0..3, g =
+ * 0..3; chains 64 w .. 64 w + 63 meet in a tree of neighbours (1, 2, 4 .. 32
+ * apart), the four results are added in order. That is what the fp32 MFMA
+ * does: 16x16x4 equals a chain of fmas over its four lane groups bit for bit
+ * (checked over 10^6 outputs), lane group g holding elements 4 g .. 4 g + 3 as
+ * loaded. The reference sums sequentially (and expf/log1pf come from ROCm's
+ * libm), so scores match within fp32 rounding, not bitwise. dim % 256 == 0,
+ * dim <= 8192.
+ *
+ * Up to 8 tokens: one workgroup per expert, its gate row in registers (thread
+ * i: chain i). */
 #define APUS_ROUTER_TT 8
+__device__ __forceinline__ void apus_router_store(float d, size_t o, float bias_e, float *sp, float *biased) {
+    const float v = d > 20.0f ? d : log1pf(expf(d));
+    const float r = sqrtf(v);
+    sp[o] = r;
+    if (biased) biased[o] = r + bias_e;
+}
+
 __global__ __launch_bounds__(256) void apus_router_kernel(
     const float *__restrict__ gate_w, const float *__restrict__ bias,
     const float *__restrict__ x, int s, int dim, int E, float *__restrict__ sp,
@@ -348,27 +364,35 @@ __global__ __launch_bounds__(256) void apus_router_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int e = blockIdx.x, t0 = blockIdx.y * APUS_ROUTER_TT;
     const int nt = min(APUS_ROUTER_TT, s - t0);
-    const int n4 = dim >> 2;
-    const float4 *wr = reinterpret_cast<const float4 *>(gate_w + (size_t)e * dim);
-    float4 g[8];
+    const int nb = dim >> 4;
+    const float *wr = gate_w + (size_t)e * dim;
+    float4 gv[2][4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-        g[i] = (tid + 256 * i < n4) ? apus_gld<float4>(wr + tid + 256 * i)
-                                    : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            gv[i][g] = (tid + 256 * i < nb) ? apus_gld<float4>(wr + (tid + 256 * i) * 16 + 4 * g)
+                                            : make_float4(0.f, 0.f, 0.f, 0.f);
     float acc[APUS_ROUTER_TT];
 #pragma unroll
     for (int t = 0; t < APUS_ROUTER_TT; ++t) {
         acc[t] = 0.0f;
         if (t < nt) {
-            const float4 *xr = reinterpret_cast<const float4 *>(x + (size_t)(t0 + t) * dim);
+            const float *xr = x + (size_t)(t0 + t) * dim;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                if (tid + 256 * i < n4) {
-                    const float4 a = apus_gld<float4>(xr + tid + 256 * i);
-                    acc[t] = acc[t] + a.x * g[i].x;
-                    acc[t] = acc[t] + a.y * g[i].y;
-                    acc[t] = acc[t] + a.z * g[i].z;
-                    acc[t] = acc[t] + a.w * g[i].w;
+            for (int i = 0; i < 2; ++i) {
+                if (tid + 256 * i < nb) {
+                    float4 a[4];
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) a[g] = apus_gld<float4>(xr + (tid + 256 * i) * 16 + 4 * g);
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) acc[t] = __builtin_fmaf(a[g].x, gv[i][g].x, acc[t]);
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) acc[t] = __builtin_fmaf(a[g].y, gv[i][g].y, acc[t]);
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) acc[t] = __builtin_fmaf(a[g].z, gv[i][g].z, acc[t]);
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) acc[t] = __builtin_fmaf(a[g].w, gv[i][g].w, acc[t]);
                 }
             }
         }
@@ -377,29 +401,20 @@ __global__ __launch_bounds__(256) void apus_router_kernel(
 #pragma unroll
     for (int t = 0; t < APUS_ROUTER_TT; ++t) {
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) acc[t] = acc[t] + __shfl_xor(acc[t], off, 64);
+        for (int off = 1; off <= 32; off <<= 1) acc[t] = acc[t] + __shfl_xor(acc[t], off, 64);
         if (lane == 0) part[wv][t] = acc[t];
     }
     __syncthreads();
-    if (tid < nt) {
-        const float d = ((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid];
-        const float v = d > 20.0f ? d : log1pf(expf(d));
-        const float r = sqrtf(v);
-        const size_t o = (size_t)(t0 + tid) * E + e;
-        sp[o] = r;
-        if (biased) biased[o] = r + bias[e];
-    }
+    if (tid < nt)
+        apus_router_store(((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid],
+                          (size_t)(t0 + tid) * E + e, biased ? bias[e] : 0.0f, sp, biased);
 }
 
-/* The same scores for more than 8 tokens: one workgroup per (8 experts, 8
- * tokens), so each gate row and each x row is read by s/8 and E/8 workgroups
- * instead of every x row by all E. Thread i takes the same K elements in the
- * same order as above (float4s i, i + 256, ...) for its 64 (expert, token)
- * dots; the xor-shuffle tree is computed as a reduce-scatter (at each step a
- * lane adds its partner's half of the values it keeps, so after six steps
- * lane l holds dot l, every addition the one the tree makes), then the four
- * wave sums in wave order: every score equals the one-expert kernel's bit for
- * bit. dim % 1024 == 0, dim <= 8192, E % 8 == 0. */
+/* A decode batch of more tokens: 8 experts x 8 tokens a workgroup, so that each
+ * gate row is read s / 8 times and each x row E / 8 times; thread i makes chain
+ * i of the 64 dots. The tree is computed as a reduce-scatter: at each step a
+ * lane adds its partner's half of the dots it keeps, so after six steps lane l
+ * holds dot bitrev(l), every addition the one the tree makes. E % 8 == 0. */
 __global__ __launch_bounds__(256) void apus_router8_kernel(
     const float *__restrict__ gate_w, const float *__restrict__ bias,
     const float *__restrict__ x, int s, int dim, int E, float *__restrict__ sp,
@@ -410,28 +425,34 @@ __global__ __launch_bounds__(256) void apus_router8_kernel(
     float v[EG * TT];                                     /* index i * TT + t */
 #pragma unroll
     for (int q = 0; q < EG * TT; ++q) v[q] = 0.0f;
-    for (int k = tid * 4; k < dim; k += 1024) {
-        float4 g[EG], a[TT];
-#pragma unroll
-        for (int i = 0; i < EG; ++i) g[i] = apus_gld<float4>(gate_w + (size_t)(e0 + i) * dim + k);
+    for (int b = tid; b < dim >> 4; b += 256) {
+        float4 a[TT][4];
 #pragma unroll
         for (int t = 0; t < TT; ++t)
-            a[t] = apus_gld<float4>(x + (size_t)min(t0 + t, s - 1) * dim + k);
 #pragma unroll
-        for (int i = 0; i < EG; ++i)
+            for (int g = 0; g < 4; ++g)
+                a[t][g] = apus_gld<float4>(x + (size_t)min(t0 + t, s - 1) * dim + b * 16 + 4 * g);
+#pragma unroll
+        for (int i = 0; i < EG; ++i) {
+            float4 w[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) w[g] = apus_gld<float4>(gate_w + (size_t)(e0 + i) * dim + b * 16 + 4 * g);
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
                 float &c = v[i * TT + t];
-                c = c + a[t].x * g[i].x;
-                c = c + a[t].y * g[i].y;
-                c = c + a[t].z * g[i].z;
-                c = c + a[t].w * g[i].w;
-            }
-    }
-    /* reduce-scatter over the wave: step `off` keeps the upper half of the
-     * remaining values in lanes with that bit set, the lower half elsewhere */
 #pragma unroll
-    for (int off = 32, n = 64; off >= 1; off >>= 1, n >>= 1) {
+                for (int g = 0; g < 4; ++g) c = __builtin_fmaf(a[t][g].x, w[g].x, c);
+#pragma unroll
+                for (int g = 0; g < 4; ++g) c = __builtin_fmaf(a[t][g].y, w[g].y, c);
+#pragma unroll
+                for (int g = 0; g < 4; ++g) c = __builtin_fmaf(a[t][g].z, w[g].z, c);
+#pragma unroll
+                for (int g = 0; g < 4; ++g) c = __builtin_fmaf(a[t][g].w, w[g].w, c);
+            }
+        }
+    }
+#pragma unroll
+    for (int off = 1, n = 64; off <= 32; off <<= 1, n >>= 1) {
         const bool up = lane & off;
 #pragma unroll
         for (int j = 0; j < n / 2; ++j) {
@@ -441,29 +462,198 @@ __global__ __launch_bounds__(256) void apus_router8_kernel(
         }
     }
     __shared__ float part[4][EG * TT];
-    part[wv][lane] = v[0];                                /* dot `lane` */
+    part[wv][__brev((unsigned)lane) >> 26] = v[0];
     __syncthreads();
     if (tid < EG * TT) {
-        const int i = tid / TT, t = tid % TT;
-        if (t0 + t < s) {
-            const float d = ((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid];
-            const float u = d > 20.0f ? d : log1pf(expf(d));
-            const float r = sqrtf(u);
-            const size_t o = (size_t)(t0 + t) * E + e0 + i;
-            sp[o] = r;
-            if (biased) biased[o] = r + bias[e0 + i];
+        const int e = e0 + tid / TT, t = t0 + tid % TT;
+        if (t < s)
+            apus_router_store(((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid], (size_t)t * E + e,
+                              biased ? bias[e] : 0.0f, sp, biased);
+    }
+}
+
+/* Prompts: fp32 MFMAs. A workgroup of 4 SW waves owns 16 TM tokens x 16 TN
+ * experts, wave w chains NC w .. NC w + NC - 1 (NC = 64 / SW) of every dot: two
+ * blocks of 16 elements a step, both operands global -> LDS into a wave-private ring PD steps deep (8
+ * rows of 128 bytes a load, chunks XOR-swizzled by row); the tree's open
+ * branches are kept a level each. 4096 tokens, 256 experts, dim 4096, beside the
+ * shared expert: 421 us on the vector units (8 x 8 dots a workgroup) -> 154, of
+ * which the MFMAs take 55 at their peak rate. */
+template <int TM, int TN, int PD, int SW>
+__global__ __launch_bounds__(256 * SW) void apus_router_mfma_kernel(
+    const float *__restrict__ gate_w, const float *__restrict__ bias,
+    const float *__restrict__ x, int s, int dim, int E, float *__restrict__ sp,
+    float *__restrict__ biased) {
+    constexpr int NL = 2 * (TM + TN), STB = NL * 1024, NC = 64 / SW, LV = SW == 1 ? 5 : SW == 2 ? 4 : 3;
+    extern __shared__ __align__(16) uint8_t rlds[];                      /* 4 SW rings; then the sums */
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int e0 = blockIdx.x * 16 * TN, t0 = blockIdx.y * 16 * TM;
+    uint8_t *ring = rlds + wave * PD * STB;
+    const unsigned rbase = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)ring);
+    const float *src[NL];
+#pragma unroll
+    for (int u = 0; u < NL; ++u) {
+        const int i = 8 * u + (lane >> 3), c = (lane & 7) ^ (i & 7);
+        src[u] = u < 2 * TM ? x + (size_t)min(t0 + i, s - 1) * dim + 4 * c
+                            : gate_w + (size_t)min(e0 + i - 16 * TM, E - 1) * dim + 4 * c;
+        src[u] += wave * (NC * 16);
+    }
+    /* this wave's steps: n0 over the blocks below 256, n1 over the rest, step
+     * s of both parts in a row */
+    const int nb = dim >> 4;
+    const int n0 = min(max(nb - NC * wave, 0), NC) >> 1, n1 = min(max(nb - 256 - NC * wave, 0), NC) >> 1;
+    const int own = n0 + n1;
+    auto issue = [&](int idx, int slot) {
+        const int st = idx < 2 * n1 ? idx >> 1 : idx - n1, part = idx < 2 * n1 ? idx & 1 : 0;
+        const int k = 32 * st + 4096 * part;
+#pragma unroll
+        for (int u = 0; u < NL; ++u) apus_g2lds16(src[u] + k, rbase + slot * STB + u * 1024);
+    };
+#pragma unroll
+    for (int d = 0; d < PD; ++d)
+        if (d < own) issue(d, d);
+    apus_v4f br[LV][TM][TN] = {}, top[TM][TN] = {}, acc[2][TM][TN] = {};
+    for (int c = 0; c < own; ++c) {
+        const int later = min(own - 1 - c, PD - 1);
+        if (PD > 2 && later >= 2) apus_wait_vm<2 * NL>();
+        else if (later == 1) apus_wait_vm<NL>();
+        else apus_wait_vm<0>();
+        const uint8_t *stg = ring + (c % PD) * STB;
+        float4 fa[2][TM], fb[2][TN];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                fa[h][i] = *reinterpret_cast<const float4 *>(stg + (16 * i + r) * 128 + (((4 * h + g) ^ (r & 7)) << 4));
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                fb[h][j] = *reinterpret_cast<const float4 *>(stg + (16 * (TM + j) + r) * 128 +
+                                                             (((4 * h + g) ^ (r & 7)) << 4));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");               /* slot read before its refill */
+        if (c + PD < own) issue(c + PD, c % PD);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        const float4 &a = fa[h][i], &b = fb[h][j];
+                        acc[h][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            q == 0 ? a.x : q == 1 ? a.y : q == 2 ? a.z : a.w,
+                            q == 0 ? b.x : q == 1 ? b.y : q == 2 ? b.z : b.w, acc[h][i][j], 0, 0, 0);
+                    }
+        if (c < 2 * n1 && !(c & 1)) continue;                            /* the chains go on in the next step */
+        /* the two chains meet; branches of equal size above them as they close */
+        const int st = c < 2 * n1 ? c >> 1 : c - n1;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                top[i][j] = acc[0][i][j] + acc[1][i][j];
+                acc[0][i][j] = acc[1][i][j] = apus_v4f{0.f, 0.f, 0.f, 0.f};
+            }
+        bool open = true;
+#pragma unroll
+        for (int lv = 0; lv < LV; ++lv) {
+            if (!open) continue;
+            const bool close = (st >> lv) & 1;
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    if (close) top[i][j] = br[lv][i][j] + top[i][j];
+                    else       br[lv][i][j] = top[i][j];
+                }
+            open = close;
         }
     }
+    /* fewer chains than that (dim < 4096): the branches left open, smallest
+     * first (the missing ones are zero) */
+    if (n0 < NC / 2) {
+        bool any = false;
+#pragma unroll
+        for (int lv = 0; lv < LV; ++lv) {
+            if (!((n0 >> lv) & 1)) continue;
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) top[i][j] = any ? br[lv][i][j] + top[i][j] : br[lv][i][j];
+            any = true;
+        }
+    }
+    __syncthreads();                                                     /* the rings become the sums' space */
+    apus_v4f *red = reinterpret_cast<apus_v4f *>(rlds);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) red[(wave * TM * TN + i * TN + j) * 64 + lane] = top[i][j];
+    __syncthreads();
+    /* lane holds D[4g + q][r]: token 16 i + 4 g + q, expert 16 j + r */
+    for (int u = threadIdx.x; u < TM * TN * 64; u += 256 * SW) {
+        const int tile = u >> 6, l = u & 63;
+        apus_v4f p[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {                                    /* the tree's last levels */
+            apus_v4f q[SW];
+#pragma unroll
+            for (int k = 0; k < SW; ++k) q[k] = red[(w * SW + k) * TM * TN * 64 + u];
+#pragma unroll
+            for (int n = 1; n < SW; n *= 2)
+#pragma unroll
+                for (int k = 0; k < SW; k += 2 * n) q[k] += q[k + n];
+            p[w] = q[0];
+        }
+        const apus_v4f d = ((p[0] + p[1]) + p[2]) + p[3];
+        const int e = e0 + 16 * (tile % TN) + (l & 15), t = t0 + 16 * (tile / TN) + 4 * (l >> 4);
+        if (e < E) {
+            const float be = biased ? bias[e] : 0.0f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (t + q < s) apus_router_store(d[q], (size_t)(t + q) * E + e, be, sp, biased);
+        }
+    }
+}
+
+template <int TM, int TN, int PD, int SW>
+hipError_t apus_launch_router_mfma(const float *gate_w, const float *bias, const float *x, int s, int dim, int E,
+                                   float *sp, float *biased, hipStream_t st) {
+    constexpr int lds = 4 * SW * PD * 2 * (TM + TN) * 1024;              /* at least the sums' space */
+    static_assert(PD * 2 * (TM + TN) >= TM * TN, "sums");
+    static const hipError_t attr = hipFuncSetAttribute(
+        reinterpret_cast<const void *>(&apus_router_mfma_kernel<TM, TN, PD, SW>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL((apus_router_mfma_kernel<TM, TN, PD, SW>),
+                       dim3((E + 16 * TN - 1) / (16 * TN), (s + 16 * TM - 1) / (16 * TM)), dim3(256 * SW), lds, st,
+                       gate_w, bias, x, s, dim, E, sp, biased);
+    return hipGetLastError();
 }
 
 hipError_t apus_launch_router(const float *gate_w, const float *bias, const float *x, int s,
                               int dim, int E, float *sp, float *biased, hipStream_t st) {
     if (s <= 0) return hipSuccess;
     if (dim % 256 || dim > 8192 || E <= 0) return hipErrorInvalidValue;
-    if (s > APUS_ROUTER_TT && dim % 1024 == 0 && E % 8 == 0) {
+    if (s <= APUS_ROUTER_TT) {
+        hipLaunchKernelGGL(apus_router_kernel, dim3(E, 1), dim3(256), 0, st, gate_w, bias, x, s, dim, E, sp, biased);
+        return hipGetLastError();
+    }
+    /* up to 64 16 x 16 tiles (a quarter of the CUs, each reading 512 KB) the vector
+     * kernel's 256 KB a workgroup over more CUs is sooner done: sublayer of 64
+     * tokens 437-443 us with it, 443-445 with the MFMAs */
+    if (E % 8 == 0 && (size_t)((s + 15) / 16) * ((E + 15) / 16) <= 64) {
         hipLaunchKernelGGL(apus_router8_kernel, dim3(E / 8, (s + APUS_ROUTER_TT - 1) / APUS_ROUTER_TT),
                            dim3(256), 0, st, gate_w, bias, x, s, dim, E, sp, biased);
         return hipGetLastError();
+    }
+    /* 16-byte loads straight to LDS: rows have to be 16-byte aligned */
+    if (((reinterpret_cast<uintptr_t>(gate_w) | reinterpret_cast<uintptr_t>(x)) & 15) == 0) {
+        if ((size_t)((s + 31) / 32) * ((E + 31) / 32) >= 256)
+            return apus_launch_router_mfma<2, 2, 2, 1>(gate_w, bias, x, s, dim, E, sp, biased, st);
+        return apus_launch_router_mfma<1, 1, 2, 4>(gate_w, bias, x, s, dim, E, sp, biased, st);
     }
     hipLaunchKernelGGL(apus_router_kernel, dim3(E, (s + APUS_ROUTER_TT - 1) / APUS_ROUTER_TT),
                        dim3(256), 0, st, gate_w, bias, x, s, dim, E, sp, biased);

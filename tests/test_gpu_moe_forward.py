@@ -280,3 +280,23 @@ def test_moe_forward_dev_graph_replays(hip, oracle, store1, rng):
         assert np.array_equal(got.view(np.uint32), eager.view(np.uint32))
         run()                                   # eager work between replays
         hip._check(L.apus_hip_synchronize(), "sync")
+
+
+@pytest.mark.parametrize("E,dim,s", [(16, 256, 9), (40, 768, 33), (24, 2048, 17), (16, 4096, 50), (16, 5120, 20),
+                                     (16, 8192, 33), (256, 1024, 1030),
+                                     (128, 1024, 300), (36, 4096, 300)])
+def test_router_order_bitwise(hip, store1, rng, E, dim, s):
+    """The matrix-core router (more than 8 tokens; both tile sizes, ragged
+    tokens and experts, one and two blocks a chain, waves without chains)
+    gives, bit for bit, the scores of calls of at most 8 tokens."""
+    inter, topk = 128, 4
+    cfg, shared, x = _case(rng, E, dim, inter, s, topk, 0, 1.0)
+    st = store1(E, dim, inter)
+    hip._check(hip.lib().apus_hip_store_fill_random(st, 3), "fill")
+    got = _run_device(hip, st, cfg, shared, x)[3]
+    for a in (0, 8, (s - 1) // 8 * 8):
+        part = _run_device(hip, st, cfg, shared, x[a:a + 8])[3]
+        assert np.array_equal(part.view(np.uint32), got[a:a + 8].view(np.uint32)), a
+    ref = x[:, :].astype(np.float64) @ cfg["gate_w"].astype(np.float64).T
+    ref = np.sqrt(np.where(ref > 20, ref, np.log1p(np.exp(np.minimum(ref, 20)))))
+    assert np.abs(got - ref).max() <= 4e-6 * np.abs(ref).max()
