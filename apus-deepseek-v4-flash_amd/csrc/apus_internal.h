@@ -286,6 +286,10 @@ hipError_t apus_launch_fill(uint8_t *dst, size_t n, uint64_t seed,
 /* elementwise BF16 rounding in place */
 hipError_t apus_launch_bf16_round(float *v, size_t n, hipStream_t st);
 
+/* copy by kernel (16-byte aligned, multiple of 16 bytes); src may be
+ * device-visible host memory */
+hipError_t apus_launch_copy(void *dst, const void *src, size_t bytes, hipStream_t st);
+
 /* a one-wave kernel that holds the stream for `ticks` wall-clock ticks */
 hipError_t apus_launch_delay(unsigned long long ticks, hipStream_t st);
 

@@ -1528,6 +1528,24 @@ hipError_t apus_launch_bf16_round(float *v, size_t n, hipStream_t st) {
     return hipGetLastError();
 }
 
+/* A staged upload: device-visible pinned host memory to device memory, 16 bytes
+ * a lane. */
+__global__ __launch_bounds__(256) void apus_copy_kernel(apus_v4u *__restrict__ dst, const apus_v4u *__restrict__ src,
+                                                        unsigned n) {
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+hipError_t apus_launch_copy(void *dst, const void *src, size_t bytes, hipStream_t st) {
+    if (!bytes) return hipSuccess;
+    if (((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src) | bytes) & 15) || bytes > (1u << 30))
+        return hipErrorInvalidValue;
+    const unsigned n = (unsigned)(bytes / 16);
+    hipLaunchKernelGGL(apus_copy_kernel, dim3((n + 255) / 256), dim3(256), 0, st, (apus_v4u *)dst,
+                       (const apus_v4u *)src, n);
+    return hipGetLastError();
+}
+
 /* ------------------------------------------------------------ delay */
 
 /* One wave that sleeps until `ticks` of the constant-rate wall clock have

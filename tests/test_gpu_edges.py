@@ -157,6 +157,27 @@ def test_nonfinite_activation_refused(hip, bad):
         hip.act_quant(x)
 
 
+@pytest.mark.parametrize("pos", [0, 2047, 2048, 4095, 6 * 1024 - 1])
+def test_nonfinite_activation_refused_at(hip, pos):
+    """The scan's blocks of 2048: their edges and a last, partial block; the
+    message names the first bad element."""
+    x = acts(np.random.default_rng(7), 6, 1024)
+    x.reshape(-1)[pos:] = np.nan
+    with pytest.raises(hip.ApusHipError, match=f"non-finite activation at element {pos} "):
+        hip.act_quant(x)
+
+
+@pytest.mark.parametrize("M,K", [(1, 128), (3, 256), (64, 4096), (65, 4096)])
+def test_upload_sizes(hip, oracle, M, K):
+    """Staged uploads from one copy block up to the largest staged size, and
+    one past it, each with new contents at once after the last call."""
+    rng = np.random.default_rng(8)
+    for _ in range(3):
+        x = acts(rng, M, K)
+        for got, want in zip(hip.act_quant(x), oracle.act_quant(x)):
+            assert np.array_equal(got, want)
+
+
 def test_nonfinite_activation_dev(hip, oracle):
     K, O = 256, 128
     rng = np.random.default_rng(6)
