@@ -14,6 +14,9 @@
  *  - prefill (apus_gemm_prefill_kernel): grouped launches with many rows
  *    per entry; activation slices double-buffered in LDS, 4 token tiles per
  *    weight pass.
+ *  - block (apus_block_loop): large tiles, both operands through LDS; dense
+ *    GEMMs of many rows, and the routed w1/w3 with SwiGLU at many rows.
+ *  - narrow (apus_gemm_narrow_kernel): dense FP8 GEMMs of 9..64 rows.
  *  - stream (apus_gemm_stream_kernel): other grouped shapes.
  * In all of them, every output is one accumulation chain over its 128-groups
  * in a fixed order, so results do not depend on M, on the position of a row
