@@ -815,7 +815,7 @@ int moe_pipeline(int E, int dim, int inter, float limit, uint8_t *const *tab,
      * 900 / 848, 1024 723 / 697; 512 605-611 / 603-609, 130 x top-8 540 / 548:
      * with fewer rows an expert the weights bound both, and the few-row
      * experts' h costs a launch over their table */
-    const bool block = use_items && wtiled && inter == 2048 && apus_moe_block_on() && (size_t)s * dim < (1ull << 32) &&
+    const bool block = use_items && wtiled && inter == 2048 && apus_moe_block_on(dim) && (size_t)s * dim < (1ull << 32) &&
                        w.n_items < 32768 && nj >= 16 * E &&
                        ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(add_src) |
                          reinterpret_cast<uintptr_t>(add_out)) & 15) == 0;

@@ -1078,23 +1078,29 @@ __global__ __launch_bounds__(512, 2) void apus_gemm_prefill_ra_kernel(ApusGemmAr
 
 /* launch the resident-activation schedule (returns false where it does not
  * apply) */
+/* whether the device takes the kernel's LDS size (asked once) */
+template <int NS, bool FOLD, bool OB>
+bool apus_pre_ra_ready() {
+    static const hipError_t attr = hipFuncSetAttribute(
+        reinterpret_cast<const void *>(&apus_gemm_prefill_ra_kernel<NS, FOLD, APUS_PRE_RA_NCB, OB>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, 64 * (2048 + 32) + 64 * (NS * 4));
+    return attr == hipSuccess;
+}
+
 template <int NS, bool FOLD>
 bool apus_launch_pre_ra(const ApusGemmArgs &p, int n_ent, hipStream_t st) {
     constexpr size_t lds = 64 * (2048 + 32) + 64 * (NS * 4);
     dim3 gr(p.O / (128 * APUS_PRE_RA_NCB), n_ent);
     auto go = [&](auto obc) {
         constexpr bool OB = obc;
-        static const hipError_t attr = hipFuncSetAttribute(
-            reinterpret_cast<const void *>(&apus_gemm_prefill_ra_kernel<NS, FOLD, APUS_PRE_RA_NCB, OB>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (attr != hipSuccess) return false;
+        if (!apus_pre_ra_ready<NS, FOLD, OB>()) return false;
         hipLaunchKernelGGL((apus_gemm_prefill_ra_kernel<NS, FOLD, APUS_PRE_RA_NCB, OB>), gr, dim3(512), lds, st, p);
         return true;
     };
     if constexpr (FOLD) {
         if (p.out_bf16) return go(std::true_type{});
     }
-    return go(std::false_type{});
+    return !p.out_bf16 && go(std::false_type{});
 }
 
 /*
@@ -3539,6 +3545,9 @@ hipError_t apus_launch_gemm_few(int wfmt, const ApusGemmArgs *a, int n_ent, int 
         (a->asrc == APUS_A_SWIGLU && !apus_group_k(a->K)) ||
         (a->acc_y && (!a->pidx || a->nmat != 1 || !a->tickets)) || ks < 0 || ks > 4 || ks == 3)
         return hipErrorInvalidValue;
+    /* BF16 outputs: the K-quarter order from codes only */
+    if (a->out_bf16 && (wfmt != APUS_W_FP4 || a->asrc != APUS_A_CODES || a->kchain != 4 || a->acc_y))
+        return hipErrorInvalidValue;
     /* two by-value entries share their activation rows (staged once, before
      * the entry lookup) */
     if (!a->ents && !a->pidx &&
@@ -3605,7 +3614,22 @@ hipError_t apus_launch_gemm_few(int wfmt, const ApusGemmArgs *a, int n_ent, int 
     return hipGetLastError();
 }
 
-bool apus_moe_block_on() { return apus_pre_lds_mode() == 1; }
+template <int NQ>
+hipError_t apus_moe_w13_attr() {
+    static const hipError_t attr = hipFuncSetAttribute(
+        reinterpret_cast<const void *>(&apus_moe_w13_block_kernel<NQ>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, ApusMoeW13<NQ>::LDS);
+    return attr;
+}
+
+/* the kernels that the routed block path cannot do without: its w1/w3, and the
+ * many-row w2 that stores BF16 (the prefill schedule in its place does not) */
+bool apus_moe_block_on(int dim) {
+    if (apus_pre_lds_mode() != 1 || !apus_pre_ra_on() || dim % (128 * APUS_PRE_RA_NCB) ||
+        !apus_pre_ra_ready<4, true, true>())
+        return false;
+    return (dim == 4096 ? apus_moe_w13_attr<32>() : apus_moe_w13_attr<16>()) == hipSuccess;
+}
 
 hipError_t apus_launch_moe_w13_block(const uint8_t *acodes, const float *ascale, const ApusGemmEnt *ents,
                                      const int2 *items, int n_items, int K, int O, float limit, uint8_t *hc, float *hs,
@@ -3615,9 +3639,7 @@ hipError_t apus_launch_moe_w13_block(const uint8_t *acodes, const float *ascale,
     const ApusMoeBlkArgs a{acodes, ascale, ents, items, O, limit, hc, hs};
     auto go = [&](auto nqc) {
         constexpr int NQ = nqc;
-        static const hipError_t attr = hipFuncSetAttribute(
-            reinterpret_cast<const void *>(&apus_moe_w13_block_kernel<NQ>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, ApusMoeW13<NQ>::LDS);
+        const hipError_t attr = apus_moe_w13_attr<NQ>();
         if (attr != hipSuccess) return attr;
         hipLaunchKernelGGL((apus_moe_w13_block_kernel<NQ>), dim3(O / 128, n_items), dim3(512), ApusMoeW13<NQ>::LDS, st, a);
         return hipGetLastError();
@@ -3632,6 +3654,9 @@ hipError_t apus_launch_gemm(int wfmt, const ApusGemmArgs *a, int n_ent,
     const size_t row_tiles = (size_t)n_ent * ((a->O + 15) / 16);
     constexpr int R = 8;
     if (a->items && (wfmt != APUS_W_FP4 || !grouped)) return hipErrorInvalidValue;
+    /* BF16 outputs: the two w2 schedules of the routed block path only (no
+     * launch that would write fp32 in their place) */
+    if (a->out_bf16 && (wfmt != APUS_W_FP4 || !grouped || a->kchain != 4 || a->K != 2048)) return hipErrorInvalidValue;
     if (a->wtiled) {
         /* tiled weights: only the decode, prefill and tile schedules read them */
         if (!(grouped ? apus_group_k(a->K) : apus_fast_k(a->K)) || a->O % 128)
@@ -3687,7 +3712,7 @@ hipError_t apus_launch_gemm(int wfmt, const ApusGemmArgs *a, int n_ent,
              * there; APUS_HIP_PRE_LDS=2 runs it for w2 as well) */
             if (a->items && a->wtiled && TT4 == 4 && apus_pre_lds_on()) {
                 bool ok = false;
-                if (a->kchain == 4) ok = apus_pre_lds_mode() == 2 && a->K == 2048 && apus_launch_pre_lds<4, true>(p, n_ent, st);
+                if (a->kchain == 4) ok = apus_pre_lds_mode() == 2 && a->K == 2048 && !a->out_bf16 && apus_launch_pre_lds<4, true>(p, n_ent, st);
                 else ok = a->K == 4096 ? apus_launch_pre_lds<8, false>(p, n_ent, st)
                                        : apus_launch_pre_lds<4, false>(p, n_ent, st);
                 if (ok) return hipGetLastError();
@@ -3696,6 +3721,7 @@ hipError_t apus_launch_gemm(int wfmt, const ApusGemmArgs *a, int n_ent,
                 if (a->K == 4096) {
                     hipLaunchKernelGGL((apus_gemm_prefill_kernel<APUS_W_FP4, 8, TT4, APUS_PRE_PD4, true>), gp, bp, 0, st, p);
                 } else if (!(ra && apus_launch_pre_ra<4, true>(p, n_ent, st))) {
+                    if (a->out_bf16) return hipErrorInvalidValue;
                     hipLaunchKernelGGL((apus_gemm_prefill_kernel<APUS_W_FP4, 4, TT4, APUS_PRE_PD4, true>), gp, bp, 0, st, p);
                 }
             } else if (ra && apus_pre_ra_w13()) {

@@ -207,10 +207,11 @@ hipError_t apus_launch_swiglu_quant_ents(const ApusGemmEnt *ents, int n_ent, con
 hipError_t apus_launch_moe_w13_block(const uint8_t *acodes, const float *ascale, const ApusGemmEnt *ents,
                                      const int2 *items, int n_items, int K, int O, float limit, uint8_t *hc, float *hs,
                                      hipStream_t st);
-/* whether the routed dispatch uses it (APUS_HIP_PRE_LDS=0 turns it off: the
- * resident-activation and prefill schedules on fp32 g, u and eo, identical
- * results) */
-bool apus_moe_block_on();
+/* whether the routed dispatch can use it, with the w2 schedule that stores BF16
+ * (APUS_HIP_PRE_LDS other than 1 or APUS_HIP_PRE_RA=0 turns it off, and so does
+ * a device that refuses a kernel's LDS size: the other many-row schedules on
+ * fp32 g, u and eo, identical results) */
+bool apus_moe_block_on(int dim);
 
 /* Counting sort of the routed pairs by expert and GEMM entry tables.
  * idx [nj] (nj = s * topk) expert ids in [0, E), E <= 1024; writes

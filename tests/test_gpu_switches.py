@@ -7,9 +7,9 @@ outputs with a child run without switches:
 
 * APUS_HIP_PRE_LDS=0 / 2 (many-row w1/w3 work items on the resident-
   activation schedule instead of the LDS one / the w2 ones on the LDS
-  schedule too), with APUS_HIP_PRE_RA=0 /
-  APUS_HIP_PRE_RA13=0 as well (many-row w2 / w1-w3 on the double-buffered
-  prefill schedule),
+  schedule too), APUS_HIP_PRE_RA=0 / APUS_HIP_PRE_RA13=0 (many-row w2 /
+  w1-w3 on the double-buffered prefill schedule), alone (the first turns the
+  block path with its BF16 expert outputs off) and with APUS_HIP_PRE_LDS=0,
   APUS_HIP_PAIR13_WIDE=0 / 1 (narrow or wide one-token w1/w3 workgroups),
   APUS_HIP_MOE_PAIRS=0 / 64 (always sort by expert / per-pair kernels up to
   64 pairs), APUS_HIP_MOE_SIDE=0 (the shared expert on the caller's stream),
@@ -81,6 +81,7 @@ def _same(a, b):
 CASES = [{"APUS_HIP_PRE_LDS": "0"}, {"APUS_HIP_PRE_LDS": "2"},
          {"APUS_HIP_PRE_LDS": "0", "APUS_HIP_PRE_RA": "0"},
          {"APUS_HIP_PRE_LDS": "0", "APUS_HIP_PRE_RA13": "0"},
+         {"APUS_HIP_PRE_RA": "0"}, {"APUS_HIP_PRE_RA13": "0"},
          {"APUS_HIP_PAIR13_WIDE": "0"}, {"APUS_HIP_PAIR13_WIDE": "1"},
          {"APUS_HIP_MOE_PAIRS": "0"}, {"APUS_HIP_MOE_PAIRS": "64"},
          {"APUS_HIP_MOE_SIDE": "0"}, {"APUS_HIP_LAYER1": "0"},
