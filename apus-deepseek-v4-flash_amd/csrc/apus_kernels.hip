@@ -985,12 +985,13 @@ __global__ __launch_bounds__(256) void apus_head_kernel(const uint16_t *__restri
  *
  * Products are exact in fp32 and sums are fp32:
  * - BF16 weights, x rounded to BF16 (flag 1): one BF16 MFMA;
- * - BF16 weights, fp32 x: three BF16 pieces that add up to x exactly, one
- *   MFMA each;
+ * - BF16 weights, fp32 x: three BF16 pieces that add up to x exactly (below
+ *   2^-110 to within 2^-134, half the least BF16), one MFMA each;
  * - FP32 weights: the fp32 MFMA (16x16x4).
  * Chains are short, for accuracy: BF16 ones are flushed into a second
- * accumulator every FL steps, the small pieces in a chain of their own, FP32
- * ones are 8 products long. Error against 64 bits at K = 1000 / 2048 / 4096:
+ * accumulator every FL steps, FP32 ones are 8 products long. The small pieces
+ * have a chain of their own over all steps (a 2^-8 of the sum, and so of its
+ * rounding). Error against 64 bits at K = 1000 / 2048 / 4096:
  * BF16 0.80 / 0.85 / 0.90e-7, FP32 0.91 / 0.99 / 1.12e-7, where
  * apus_wgemv_kernel's lane chains give 0.99 / 1.23 / 1.59e-7.
  *
@@ -1054,6 +1055,16 @@ __device__ __forceinline__ void apus_bf16_pieces(const float (&v)[8], apus_v8bf 
         out[p] = __builtin_bit_cast(apus_v8bf, apus_v4u{q[p][0], q[p][1], q[p][2], q[p][3]});
 }
 
+/* The small pieces' sum as it is added to the rest: an infinite weight leaves
+ * NaN there (its product with a piece that is zero) or an infinity of either
+ * sign, while the first pieces' sum holds what the product of x itself is. So
+ * what is not finite is made +-FLT_MAX, which moves no infinity. */
+__device__ __forceinline__ apus_v4f apus_small_sum(const apus_v4f &v) {
+    constexpr float big = 3.402823466e38f;
+    return apus_v4f{__builtin_amdgcn_fmed3f(v.x, -big, big), __builtin_amdgcn_fmed3f(v.y, -big, big),
+                    __builtin_amdgcn_fmed3f(v.z, -big, big), __builtin_amdgcn_fmed3f(v.w, -big, big)};
+}
+
 template <bool WB, int P, int TM, int TN, int PD, int NW>
 __global__ __launch_bounds__(64 * NW) void apus_wgemm_kernel(const void *__restrict__ w,
                                                          const float *__restrict__ x,
@@ -1105,7 +1116,7 @@ __global__ __launch_bounds__(64 * NW) void apus_wgemm_kernel(const void *__restr
             }
         }
     };
-    /* chains: BF16 [0] of the (first) pieces, [1] of the small pieces */
+    /* chains: BF16 [0] of the (first) pieces, [1] of the small pieces, never flushed */
     apus_v4f acc[2][TM][TN] = {}, tot[TM][TN] = {};
     const int nst = (K + 31) >> 5;
     const int own = wave < nst ? (nst - wave + NW - 1) / NW : 0;         /* this wave's steps */
@@ -1204,8 +1215,8 @@ __global__ __launch_bounds__(64 * NW) void apus_wgemm_kernel(const void *__restr
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
-                    tot[i][j] += P > 1 ? acc[0][i][j] + acc[1][i][j] : acc[0][i][j];
-                    acc[0][i][j] = acc[1][i][j] = apus_v4f{0.f, 0.f, 0.f, 0.f};
+                    tot[i][j] += acc[0][i][j];
+                    acc[0][i][j] = apus_v4f{0.f, 0.f, 0.f, 0.f};
                 }
         }
     }
@@ -1214,7 +1225,9 @@ __global__ __launch_bounds__(64 * NW) void apus_wgemm_kernel(const void *__restr
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) red[(wave * TM * TN + i * TN + j) * 64 + lane] = tot[i][j] + (acc[0][i][j] + acc[1][i][j]);
+        for (int j = 0; j < TN; ++j)
+            red[(wave * TM * TN + i * TN + j) * 64 + lane] =
+                P > 1 ? (tot[i][j] + acc[0][i][j]) + apus_small_sum(acc[1][i][j]) : tot[i][j] + acc[0][i][j];
     __syncthreads();
     /* lane holds D[4g + q][r]: x row 16 i + 4 g + q, weight row 16 j + r */
     for (int e = threadIdx.x; e < TM * TN * 64; e += 64 * NW) {

@@ -154,3 +154,36 @@ def test_many_rows_unaligned(hip, oracle, rng):
     hip._check(L.apus_hip_wlinear_dev(dw.ptr, dx.ptr + 4, do.ptr, M, K, O, 0), "wlinear")
     hip._check(L.apus_hip_synchronize(), "sync")
     _check(do.to_array(np.float32, (M, O)), oracle, w, x, 0)
+
+
+@pytest.mark.parametrize("flags", [0, 3, 4, 5, 6])
+def test_many_rows_non_finite_weights(hip, rng, flags):
+    """Infinite and NaN weights, on rows of x that BF16 holds exactly (their
+    small pieces are zero) and others, and on a zero of x: a 24-row call gives
+    them where three 8-row calls do, and the other outputs stay what they are
+    (1e-5 of the row's largest; one BF16 step)."""
+    M, K, O = 24, 200, 70
+    w, x = _data(rng, M, K, O, flags & 4)
+    x[::2] = (x[::2].view(np.uint32) & 0xFFFF0000).view(np.float32)
+    x[3, 5] = 0.0
+    inf, nan = ((0x7F80, 0x7FC0) if flags & 4 else (np.float32(np.inf), np.float32(np.nan)))
+    w[2, 5], w[17, 199], w[40, 31] = inf, (0xFF80 if flags & 4 else -inf), nan
+    w[69, 64], w[69, 65] = inf, inf
+    L = hip.lib()
+    dw, dx = hip.DevBuf.from_array(w), hip.DevBuf.from_array(x)
+    outs = []
+    for rows in (24, 8):
+        do = hip.DevBuf(M * O * 4)
+        for m in range(0, M, rows):
+            hip._check(L.apus_hip_wlinear_dev(dw.ptr, dx.ptr + m * K * 4, do.ptr + m * O * 4, rows, K, O,
+                                              flags), "wlinear")
+        hip._check(L.apus_hip_synchronize(), "sync")
+        outs.append(do.to_array(np.float32, (M, O)))
+    a, b = (v.astype(np.float64) for v in outs)
+    assert np.isinf(b[:, 2]).sum() == M - 1 and np.isnan(b[3, 2]) and np.isnan(b[:, 40]).all()
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
+    assert np.array_equal(a[np.isinf(a)], b[np.isinf(b)])
+    fin = np.isfinite(a)
+    scale = np.where(fin, np.abs(b), 0).max(1, keepdims=True)
+    d = np.abs(np.where(fin, a, 0) - np.where(fin, b, 0))
+    assert (d <= (2.0 ** -7 if flags & 2 else 1e-5) * scale).all()
