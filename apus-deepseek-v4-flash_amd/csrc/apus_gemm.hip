@@ -3757,10 +3757,16 @@ hipError_t apus_launch_gemm(int wfmt, const ApusGemmArgs *a, int n_ent,
 #endif
 
 #define APUS_TILE(NQ, PD) hipLaunchKernelGGL((apus_gemm_tile_kernel<WFC, NQ, (PD * APUS_TILE_PDX < NQ ? PD * APUS_TILE_PDX : NQ), APUS_TILE_DA, APUS_TILE_TM, APUS_TILE_NW(NQ)>), gt, bt, 0, st, *a)
+        /* the narrow and block schedules bring every operand by 16-byte loads
+         * straight to LDS (MXFP4 scales too; FP8 tile scales go another way);
+         * the tile schedule takes the operands that are not aligned for them */
+        const auto at16 = [](const void *v) { return (reinterpret_cast<uintptr_t>(v) & 15) == 0; };
+        const bool al16 = at16(a->ent0.w) && at16(a->acodes) && at16(a->ascale) &&
+                          (wfmt == APUS_W_FP8 || at16(a->ent0.ws));
         /* FP8 on tiled weights, plain row ranges, up to 64 rows: the narrow
          * schedule */
-        if (wfmt == APUS_W_FP8 && a->wtiled && !a->ent0.arows && !a->ent0.orows && a->ent0.M <= 64 &&
-            (reinterpret_cast<uintptr_t>(a->ascale) & 15) == 0 && apus_narrow_on()) {
+        if (wfmt == APUS_W_FP8 && a->wtiled && !a->ent0.arows && !a->ent0.orows && a->ent0.M <= 64 && al16 &&
+            apus_narrow_on()) {
             bool ok = false;
             switch (a->K) {
             case 1024: ok = apus_launch_narrow<8>(*a, st); break;
@@ -3770,10 +3776,9 @@ hipError_t apus_launch_gemm(int wfmt, const ApusGemmArgs *a, int n_ent,
             }
             if (ok) return hipGetLastError();
         }
-        /* tiled weights, plain row ranges, outputs and scales that 16-byte
-         * accesses can take: the block schedule */
-        if (a->wtiled && !a->ent0.arows && !a->ent0.orows && a->ldo % 4 == 0 &&
-            ((reinterpret_cast<uintptr_t>(a->ent0.out) | reinterpret_cast<uintptr_t>(a->ascale)) & 15) == 0 &&
+        /* tiled weights, plain row ranges, outputs that 16-byte stores can
+         * take: the block schedule */
+        if (a->wtiled && !a->ent0.arows && !a->ent0.orows && a->ldo % 4 == 0 && at16(a->ent0.out) && al16 &&
             apus_lds_tile_on()) {
             bool ok = false;
 #define APUS_BLOCK(NQ) ok = wfmt == APUS_W_FP4 ? apus_launch_block<APUS_W_FP4, NQ>(*a, st) : apus_launch_block<APUS_W_FP8, NQ>(*a, st)

@@ -98,3 +98,30 @@ def test_block_schedule_unaligned_out(hip, oracle, rng):
     got = do.to_array(np.float32, (M * O + 4,))[1:1 + M * O].reshape(M, O)
     want = gemm_tiled(hip, 1, w, ws, c, s, 1)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("what", ["w", "ws", "codes", "scales"])
+@pytest.mark.parametrize("fmt,M", [(0, 20), (0, 70), (1, 20), (1, 70)])
+def test_unaligned_operands(hip, rng, fmt, M, what):
+    """Operands at 4-byte offsets, which the narrow and block schedules' loads
+    to LDS do not take: the tile schedule, the bits of the same GEMM on
+    row-major weights."""
+    O, K = 256, 2048
+    L = hip.lib()
+    w, ws = (fp4_weights if fmt == 0 else fp8_weights)(rng, O, K)
+    c, s = hip.act_quant(acts(rng, M, K))
+    _, _, (tw, tws) = dev_pack(hip, fmt, w, ws, O, K)
+    bufs = {"w": (tw, w.nbytes), "ws": (tws, ws.nbytes) if fmt == 0 else (hip.DevBuf.from_array(ws), ws.nbytes),
+            "codes": (hip.DevBuf.from_array(c), c.nbytes), "scales": (hip.DevBuf.from_array(s), s.nbytes)}
+    b, n = bufs[what]
+    moved = hip.DevBuf(n + 16)
+    hip._check(L.apus_hip_d2d(moved.ptr + 4, b.ptr, n), "d2d")
+    ptr = {k: v[0].ptr for k, v in bufs.items()} | {what: moved.ptr + 4}
+    do = hip.DevBuf(M * O * 4)
+    fn = L.apus_hip_fp4_gemm_dev if fmt == 0 else L.apus_hip_fp8_gemm_dev
+    hip._check(fn(ptr["w"], ptr["ws"], ptr["codes"], ptr["scales"], do.ptr, M, O, K, hip.W_TILED), "gemm")
+    hip._check(L.apus_hip_synchronize(), "sync")
+    got = do.to_array(np.float32, (M, O))
+    # FP8 tile scales come by 4-byte loads: no other path for them
+    want = (gemm_tiled if fmt == 1 and what == "ws" else gemm_rows)(hip, fmt, w, ws, c, s)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
