@@ -807,16 +807,24 @@ int moe_pipeline(int E, int dim, int inter, float limit, uint8_t *const *tab,
     /* the many-row entries run from the route kernel's work list (balanced
      * row chunks) where the many-row schedules apply */
     const bool use_items = (dim == 2048 || dim == 4096) && (inter == 2048 || inter == 4096);
-    /* MXFP4 tiled experts, sixteen or more pairs an expert on average: the
-     * many-row items' w1/w3 on the block schedule, which hands w2 quantised h
-     * (its 32-bit row offsets reach 4 GiB), and eo stored as the BF16 values it
-     * holds where the schedules of w2 can (inter 2048; 16-byte rows of y).
-     * us without / with it, 256 experts, top-6: 4096 tokens 1440 / 1226, 2048
-     * 900 / 848, 1024 723 / 697; 512 605-611 / 603-609, 130 x top-8 540 / 548:
-     * with fewer rows an expert the weights bound both, and the few-row
-     * experts' h costs a launch over their table */
-    const bool block = use_items && wtiled && inter == 2048 && apus_moe_block_on(dim) && (size_t)s * dim < (1ull << 32) &&
-                       w.n_items < 32768 && nj >= 16 * E &&
+    /* MXFP4 tiled experts with many pairs: the many-row items' w1/w3 on the block
+     * schedule, which hands w2 quantised h (its 32-bit row offsets reach 4 GiB),
+     * and eo stored as the BF16 values it holds where the schedules of w2 can
+     * (inter 2048; 16-byte rows of y). It needs both pairs an expert (with fewer
+     * the weights bound either way, and the few-row experts' h costs a launch
+     * over their table) and pairs in all (a workgroup takes 128 rows x 128
+     * columns of w1 and w3, so few of them leave CUs idle). us without / with
+     * it, top-6, dim 4096, uniform routing / Zipf(1.1):
+     *   256 experts, 16 pairs each 699 / 696, 679 / 662; 96 each 1502 / 1286, 1480 / 1305
+     *   64 experts, 16 each 195 / 199, 205 / 200; 32 each 210 / 203, 231 / 230
+     *   16 experts, 64 each 92 / 84, 90 / 86; 128 each 139 / 140, 141 / 141
+     *   8 experts, 128 each 72 / 77, 71 / 77 (96 each); 256 or more 100 / 86
+     * and at dim 2048, where w1/w3 are half as long beside the same launches:
+     *   256 experts, 16 each 392 / 404; 28 each 435 / 435, 469 / 456
+     *   32 experts, 96 each 113 / 106, 110 / 113; 192 each 202 / 179, 200 / 178 */
+    const bool many = dim == 4096 ? nj >= 2048 && nj >= 16 * E : nj >= 5120 && nj >= 28 * E;
+    const bool block = use_items && wtiled && inter == 2048 && many && apus_moe_block_on(dim) &&
+                       (size_t)s * dim < (1ull << 32) && w.n_items < 32768 &&
                        ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(add_src) |
                          reinterpret_cast<uintptr_t>(add_out)) & 15) == 0;
     const int n_items128 = block ? apus_moe_items_bound(nj, E, SMALL, 128) : 0;

@@ -6,8 +6,9 @@ Usage: python tests/switch_probe.py OUT.npz
 
 Cases (all seeded, the same in every run):
 * routed dispatch over a 16-expert store at dim 4096 / inter 2048, top-6,
-  s = 1, 2, 4 (one-token and per-pair kernels) and 64 (sorted: few-row and
-  many-row schedules): y and the h codes / scale bytes of every pair;
+  s = 1, 2, 4 (one-token and per-pair kernels), 64 (sorted: few-row and
+  many-row schedules) and 352 (the block schedule): y and the h codes / scale
+  bytes of every pair;
 * the whole MoE sublayer at s = 8 (router, top-k, routed, FP8 shared
   expert, sum): out, routed, shared;
 * dense decode-schedule launches: an FP8 [4096, 4096] GEMV at M = 1 and a
@@ -111,9 +112,9 @@ def main():
     hip._check(L.apus_hip_store_fill_random(st, 31), "store fill")
     out = {}
     rng = np.random.default_rng(77)
-    for s in (1, 2, 4, 64):
+    for s in (1, 2, 4, 64, 352):
         print(f"switch_probe: routed s={s}", flush=True)
-        routed(L, st, s, rng, out)
+        routed(L, st, s, rng if s < 352 else np.random.default_rng(78), out)
     print("switch_probe: sublayer s=8", flush=True)
     sublayer(L, st, rng, out)
     print("switch_probe: dense", flush=True)

@@ -303,16 +303,18 @@ def test_routed_with_dense_rider(hip, oracle, store, rng, s):
 
 @pytest.mark.parametrize("dim", [2048, 4096])
 def test_moe_routed_block_schedule(hip, oracle, store, rng, dim):
-    """Sixteen or more pairs an expert on average take the block schedule for
-    the many-row w1/w3 (128-row and 64-row tiles: experts of 129, 128, 65, 64,
-    9 and 5 rows) and BF16 expert outputs: y and the h codes equal, bit for
-    bit, those of the same tokens dispatched in batches too small for it, and
-    the first batch passes the oracle's stage checks."""
-    E, inter, s, topk, part = 8, 2048, 200, 2, 50
+    """Many pairs take the block schedule for the many-row w1/w3 (128-row and
+    64-row tiles: experts of 129, 128, 65, 64, 9 and 5 rows, and the rest) and
+    BF16 expert outputs: y and the h codes equal, bit for bit, those of the
+    same tokens dispatched in batches too small for it, and the first batch
+    passes the oracle's stage checks."""
+    E, inter, topk, part = 8, 2048, 2, 500
+    need = 2048 if dim == 4096 else 5120       # pairs (moe_pipeline)
+    s = need // topk
     counts = [129, 128, 65, 64, 9, 5]
-    flat = rng.permutation(np.repeat(np.arange(6), counts))
+    flat = rng.permutation(np.repeat(np.arange(7), counts + [need - sum(counts)]))
     idx = flat.reshape(s, topk).astype(np.int32)
-    assert s * topk >= 16 * E > part * topk
+    assert part * topk < need and need >= 28 * E
     wgt = rng.random((s, topk)).astype(np.float32)
     x = acts(rng, s, dim)
     st = store(1, E, dim, inter)
@@ -332,12 +334,11 @@ def test_moe_routed_block_schedule(hip, oracle, store, rng, dim):
                 he.to_array(np.uint8, (n * topk, inter // 128)), wsp)
 
     y, hc, he, _ = run(0, s)
-    for a in range(0, s, part):
-        yp, hcp, hep, wsp = run(a, a + part)
-        assert np.array_equal(y[a:a + part].view(np.uint32), yp.view(np.uint32)), a
-        assert np.array_equal(hc[topk * a:topk * (a + part)], hcp), a
-        assert np.array_equal(he[topk * a:topk * (a + part)], hep), a
+    for a, b in zip([0] + list(range(50, s, part)), list(range(50, s, part)) + [s]):
+        yp, hcp, hep, wsp = run(a, b)
+        assert np.array_equal(y[a:b].view(np.uint32), yp.view(np.uint32)), a
+        assert np.array_equal(hc[topk * a:topk * b], hcp), a
+        assert np.array_equal(he[topk * a:topk * b], hep), a
         if a == 0:
-            host = {e: host_expert(oracle, 5, 0, e, E, dim, inter) for e in range(6)}
-            stage_check(hip, oracle, st, lambda e: host[e], x[:part], idx[:part], wgt[:part], yp, wsp, inter,
-                        [0, 17, 49])
+            host = {e: host_expert(oracle, 5, 0, e, E, dim, inter) for e in range(7)}
+            stage_check(hip, oracle, st, lambda e: host[e], x[:b], idx[:b], wgt[:b], yp, wsp, inter, [0, 17, 49])

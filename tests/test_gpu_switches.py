@@ -70,7 +70,7 @@ def default_run(tmp_path_factory):
     return _probe(tmp_path_factory.mktemp("switch"), "default", {})
 
 
-ROUTED = [k for s in (1, 2, 4, 64) for k in (f"y{s}", f"hc{s}", f"he{s}")] + \
+ROUTED = [k for s in (1, 2, 4, 64, 352) for k in (f"y{s}", f"hc{s}", f"he{s}")] + \
     ["fwd_out", "fwd_routed", "fwd_shared", "fwd_idx"]
 
 
