@@ -147,6 +147,18 @@ __device__ __forceinline__ void apus_g2lds4(const void *g, unsigned lds) {
 template <int N>
 __device__ __forceinline__ void apus_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
+/* 16-byte reads from LDS bytes a[i] + OFF, complete on return. For reads of a ring
+ * that loads to LDS are filling: before a read of its own the compiler, which
+ * cannot tell the slots apart, waits for every such load in flight. */
+template <int OFF>
+__device__ __forceinline__ void apus_lds_read4(apus_v4f (&d)[4], const unsigned (&a)[4]) {
+    asm volatile("ds_read_b128 %0, %4 offset:%8\n\tds_read_b128 %1, %5 offset:%8\n\t"
+                 "ds_read_b128 %2, %6 offset:%8\n\tds_read_b128 %3, %7 offset:%8\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(d[0]), "=&v"(d[1]), "=&v"(d[2]), "=&v"(d[3])
+                 : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "n"(OFF)
+                 : "memory");
+}
+
 /* 16-byte chunk slot of chunk c of a 128-byte activation row staged in LDS:
  * c ^ apus_row_swz(row). A fragment read (ds_read_b128, lane (r, g) reading
  * chunk g or 4 + g of row r, 16 rows) is then conflict-free on gfx950:

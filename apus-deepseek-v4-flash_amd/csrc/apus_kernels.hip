@@ -14,6 +14,9 @@
 #include "apus_device.h"
 #include "apus_internal.h"
 
+#include <type_traits>
+#include <utility>
+
 /* ------------------------------------------------------------ act quant */
 
 /* One wave per (row, 128-group): two elements per lane. */
@@ -411,64 +414,129 @@ __global__ __launch_bounds__(256) void apus_router_kernel(
 }
 
 /* A decode batch of more tokens: 8 experts x 8 tokens a workgroup, so that each
- * gate row is read s / 8 times and each x row E / 8 times; thread i makes chain
- * i of the 64 dots. The tree is computed as a reduce-scatter: at each step a
- * lane adds its partner's half of the dots it keeps, so after six steps lane l
- * holds dot bitrev(l), every addition the one the tree makes. E % 8 == 0. */
-__global__ __launch_bounds__(256) void apus_router8_kernel(
+ * gate row is read s / 8 times and each x row E / 8 times. KW of its four waves
+ * split K (wave k: chains 64 k .. 64 k + 63, one a lane), the others the experts.
+ * A wave brings its part of a row (4 KB) global -> LDS into a ring of four, the x
+ * rows first, which stay in registers, then the gate rows; a lane's block of 64
+ * bytes is read back as its four chunks, chunk c of lane l's block in slot
+ * c ^ (l / 4 % 4) of its four: no bank conflicts. The tree is computed as a
+ * reduce-scatter: at each step a lane adds its partner's half of the dots it
+ * keeps, every addition the one the tree makes.
+ * 256 experts, us with each lane loading its block straight from global memory
+ * (four times the cache lines a load; at dim 1024 one wave of four at work) /
+ * with this: dim 4096, 9 / 33 / 64 tokens 8.8 / 9.4 / 11.2 -> 8.0 / 8.8 / 9.0; dim
+ * 1024 6.7 / 6.6 / 7.3 -> 4.1 / 4.6 / 4.6. Bound by its fused multiply-adds (1024
+ * a lane, 1.7 us of a workgroup at dim 4096) beside the first loads' latency. */
+template <int N, class F, int... I>
+__device__ __forceinline__ void apus_unrolled_at(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+/* f(0), f(1) .. f(N - 1), each a constant */
+template <int N, class F>
+__device__ __forceinline__ void apus_unrolled(F &&f) { apus_unrolled_at<N>(f, std::make_integer_sequence<int, N>{}); }
+
+#define APUS_ROUTER8_LDS (4 * 4 * 4096)
+template <int KW>
+__global__ __launch_bounds__(256, 2) void apus_router8_kernel(
     const float *__restrict__ gate_w, const float *__restrict__ bias,
     const float *__restrict__ x, int s, int dim, int E, float *__restrict__ sp,
     float *__restrict__ biased) {
-    constexpr int EG = 8, TT = APUS_ROUTER_TT;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int e0 = blockIdx.x * EG, t0 = blockIdx.y * TT;
-    float v[EG * TT];                                     /* index i * TT + t */
+    constexpr int TT = APUS_ROUTER_TT, EW = 2 * KW, ND = EW * TT;    /* experts and dots of a wave */
+    constexpr int NR = TT + EW, NS = 4;                              /* rows of a part of K; ring */
+    static_assert(NS <= TT && 4 * NS * 4096 == APUS_ROUTER8_LDS && (KW < 4 || NR % NS == 0), "ring");
+    extern __shared__ __align__(16) uint8_t rlds[];                  /* 4 rings; then the sums */
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kw = wave % KW, eg = wave / KW;
+    const int e0 = blockIdx.x * 8 + eg * EW, t0 = blockIdx.y * TT;
+    const int nb = dim >> 4, parts = KW == 4 && nb > 256 ? 2 : 1;      /* KW < 4: nb <= 128 */
+    uint8_t *ring = rlds + wave * NS * 4096;
+    const unsigned rbase = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)ring);
+    /* load j of a row: its blocks 16 j + lane / 4; past the last block that one
+     * again (its lanes take no part) */
+    unsigned off[4];
+    auto offsets = [&](int part) {
 #pragma unroll
-    for (int q = 0; q < EG * TT; ++q) v[q] = 0.0f;
-    for (int b = tid; b < dim >> 4; b += 256) {
-        float4 a[TT][4];
+        for (int j = 0; j < 4; ++j)
+            off[j] = min(256 * part + 64 * kw + 16 * j + (lane >> 2), nb - 1) * 64 +
+                     (((lane & 3) ^ ((lane >> 4) & 3)) << 4);
+    };
+    auto issue = [&](int row) {
+        const float *p = row < TT ? x + (size_t)min(t0 + row, s - 1) * dim
+                                  : gate_w + (size_t)min(e0 + row - TT, E - 1) * dim;
 #pragma unroll
-        for (int t = 0; t < TT; ++t)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                a[t][g] = apus_gld<float4>(x + (size_t)min(t0 + t, s - 1) * dim + b * 16 + 4 * g);
-#pragma unroll
-        for (int i = 0; i < EG; ++i) {
-            float4 w[4];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) w[g] = apus_gld<float4>(gate_w + (size_t)(e0 + i) * dim + b * 16 + 4 * g);
-#pragma unroll
-            for (int t = 0; t < TT; ++t) {
-                float &c = v[i * TT + t];
-#pragma unroll
-                for (int g = 0; g < 4; ++g) c = __builtin_fmaf(a[t][g].x, w[g].x, c);
-#pragma unroll
-                for (int g = 0; g < 4; ++g) c = __builtin_fmaf(a[t][g].y, w[g].y, c);
-#pragma unroll
-                for (int g = 0; g < 4; ++g) c = __builtin_fmaf(a[t][g].z, w[g].z, c);
-#pragma unroll
-                for (int g = 0; g < 4; ++g) c = __builtin_fmaf(a[t][g].w, w[g].w, c);
-            }
+        for (int j = 0; j < 4; ++j) {
+            unsigned o = off[j];
+            asm("" : "+v"(o));                                       /* 32 bits beside the uniform base */
+            apus_g2lds16(reinterpret_cast<const uint8_t *>(p) + o, rbase + (row % NS) * 4096 + j * 1024);
         }
+    };
+    unsigned lrd[4];                                                 /* LDS bytes of the lane's four chunks in slot 0 */
+#pragma unroll
+    for (int c = 0; c < 4; ++c) lrd[c] = rbase + lane * 64 + ((c ^ ((lane >> 2) & 3)) << 4);
+    float v[ND];                                                     /* index i * TT + t */
+#pragma unroll
+    for (int q = 0; q < ND; ++q) v[q] = 0.0f;
+    offsets(0);
+#pragma unroll
+    for (int r = 0; r < NS; ++r) issue(r);
+    for (int part = 0; part < parts; ++part) {
+        const bool more = part + 1 < parts, live = 256 * part + 64 * kw + lane < nb;
+        apus_v4f a[TT][4];
+        auto row = [&](auto rc) {
+            constexpr int r = rc;
+            /* rows behind this one in flight: three, or what is left of the last part */
+            if (r + NS <= NR || more) apus_wait_vm<4 * (NS - 1)>();
+            else if (r + 3 == NR)     apus_wait_vm<8>();
+            else if (r + 2 == NR)     apus_wait_vm<4>();
+            else                      apus_wait_vm<0>();
+            apus_v4f w[4];
+            apus_lds_read4<(r % NS) * 4096>(r < TT ? a[r < TT ? r : 0] : w, lrd);
+            if (r + NS == NR) offsets(1);
+            if (r + NS < NR) issue(r + NS);
+            else if (more)   issue(r + NS - NR);
+            if (r >= TT && live) {
+#pragma unroll
+                for (int t = 0; t < TT; ++t) {
+                    float &d = v[(r < TT ? 0 : r - TT) * TT + t];
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) d = __builtin_fmaf(a[t][g].x, w[g].x, d);
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) d = __builtin_fmaf(a[t][g].y, w[g].y, d);
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) d = __builtin_fmaf(a[t][g].z, w[g].z, d);
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) d = __builtin_fmaf(a[t][g].w, w[g].w, d);
+                }
+            }
+        };
+        apus_unrolled<NR>(row);
     }
 #pragma unroll
-    for (int off = 1, n = 64; off <= 32; off <<= 1, n >>= 1) {
+    for (int off = 1, n = ND; off <= 32; off <<= 1, n = n > 1 ? n >> 1 : 1) {
         const bool up = lane & off;
+        if (n == 1) {
+            v[0] = v[0] + __shfl_xor(v[0], off, 64);
+            continue;
+        }
 #pragma unroll
         for (int j = 0; j < n / 2; ++j) {
-            const float send = up ? v[j] : v[j + n / 2];
-            const float keep = up ? v[j + n / 2] : v[j];
+            const float keep = up ? v[n / 2 + j] : v[j];
+            const float send = up ? v[j] : v[n / 2 + j];
             v[j] = keep + __shfl_xor(send, off, 64);
         }
     }
-    __shared__ float part[4][EG * TT];
-    part[wv][__brev((unsigned)lane) >> 26] = v[0];
+    /* lane l holds the dot whose bits are l's lowest ones in reverse */
+    constexpr int LB = ND == 64 ? 6 : ND == 32 ? 5 : 4;
+    __syncthreads();                                                 /* the rings become the sums' space */
+    float *red = reinterpret_cast<float *>(rlds);                    /* [KW][8 TT] */
+    if (lane < ND) red[kw * 8 * TT + eg * ND + (__brev((unsigned)lane) >> (32 - LB))] = v[0];
     __syncthreads();
-    if (tid < EG * TT) {
-        const int e = e0 + tid / TT, t = t0 + tid % TT;
-        if (t < s)
-            apus_router_store(((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid], (size_t)t * E + e,
-                              biased ? bias[e] : 0.0f, sp, biased);
+    if (threadIdx.x < 8 * TT) {
+        const int i = threadIdx.x, e = blockIdx.x * 8 + i / TT, t = t0 + i % TT;
+        float d = red[i];
+#pragma unroll
+        for (int k = 1; k < KW; ++k) d += red[k * 8 * TT + i];
+        if (t < s && e < E) apus_router_store(d, (size_t)t * E + e, biased ? bias[e] : 0.0f, sp, biased);
     }
 }
 
@@ -641,16 +709,26 @@ hipError_t apus_launch_router(const float *gate_w, const float *bias, const floa
         hipLaunchKernelGGL(apus_router_kernel, dim3(E, 1), dim3(256), 0, st, gate_w, bias, x, s, dim, E, sp, biased);
         return hipGetLastError();
     }
-    /* up to 64 16 x 16 tiles (a quarter of the CUs, each reading 512 KB) the vector
-     * kernel's 256 KB a workgroup over more CUs is sooner done: sublayer of 64
-     * tokens 437-443 us with it, 443-445 with the MFMAs */
-    if (E % 8 == 0 && (size_t)((s + 15) / 16) * ((E + 15) / 16) <= 64) {
-        hipLaunchKernelGGL(apus_router8_kernel, dim3(E / 8, (s + APUS_ROUTER_TT - 1) / APUS_ROUTER_TT),
-                           dim3(256), 0, st, gate_w, bias, x, s, dim, E, sp, biased);
-        return hipGetLastError();
-    }
     /* 16-byte loads straight to LDS: rows have to be 16-byte aligned */
     if (((reinterpret_cast<uintptr_t>(gate_w) | reinterpret_cast<uintptr_t>(x)) & 15) == 0) {
+        /* The vector kernel while each CU has one workgroup of it at most, or two
+         * with few blocks of tokens (then its gate rows are shared by few); the
+         * MFMA kernel's 16 x 16 tiles take 13 us of dim 4096 however few they are.
+         * us, dim 4096, vector / MFMA: 256 experts, 64 tokens 9.0 / 13.2, 80 12.8 /
+         * 13.6, 112 13.2 / 14.2, 128 13.8-16.1 / 14.2, 160 18.8 / 14.6; 512 experts,
+         * 64 tokens 12.5 / 13.7; 1024, 33 tokens 16.6 / 13.8; 128, 128 tokens 9.1 /
+         * 14.1, 136 13.2 / 14.0, 200 16.1 / 14.5; 64, 256 tokens 12.2 / 14.3, 257 16.8 /
+         * 14.2; 16, 1000 tokens 11.6 / 13.9 */
+        const size_t wgs = (size_t)((E + 7) / 8) * ((s + APUS_ROUTER_TT - 1) / APUS_ROUTER_TT);
+        if (wgs <= 256 || (wgs <= 512 && s <= 112)) {
+            const dim3 grid((E + 7) / 8, (s + APUS_ROUTER_TT - 1) / APUS_ROUTER_TT);
+            auto go = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, grid, dim3(256), APUS_ROUTER8_LDS, st, gate_w, bias, x, s, dim, E, sp, biased);
+                return hipGetLastError();
+            };
+            return dim > 2048 ? go(apus_router8_kernel<4>) : dim > 1024 ? go(apus_router8_kernel<2>)
+                                                                        : go(apus_router8_kernel<1>);
+        }
         if ((size_t)((s + 31) / 32) * ((E + 31) / 32) >= 256)
             return apus_launch_router_mfma<2, 2, 2, 1>(gate_w, bias, x, s, dim, E, sp, biased, st);
         return apus_launch_router_mfma<1, 1, 2, 4>(gate_w, bias, x, s, dim, E, sp, biased, st);

@@ -282,13 +282,18 @@ def test_moe_forward_dev_graph_replays(hip, oracle, store1, rng):
         hip._check(L.apus_hip_synchronize(), "sync")
 
 
-@pytest.mark.parametrize("E,dim,s", [(16, 256, 9), (40, 768, 33), (24, 2048, 17), (16, 4096, 50), (16, 5120, 20),
-                                     (16, 8192, 33), (256, 1024, 1030),
-                                     (128, 1024, 300), (36, 4096, 300)])
+@pytest.mark.parametrize("E,dim,s", [
+    # the vector kernel of 8 experts x 8 tokens: K on one, two and four waves, lanes and waves without
+    # chains, one and two blocks a chain, ragged tokens and experts
+    (16, 256, 9), (40, 768, 33), (20, 1024, 20), (24, 2048, 17), (41, 1280, 12), (16, 2304, 30), (16, 4096, 50),
+    (36, 4096, 300), (20, 4352, 20), (16, 5120, 20), (16, 8192, 33),
+    # the matrix-core kernel, 16 x 16 tiles: one and two blocks a chain, waves without chains
+    (128, 1024, 300), (200, 768, 170), (256, 4096, 130), (250, 5120, 131), (256, 8192, 137),
+    # 32 x 32 tiles: the same, and branches left open (dim not a multiple of 1024)
+    (256, 1024, 1030), (256, 768, 1030), (250, 4096, 1030), (256, 4864, 1025), (256, 5120, 1030)])
 def test_router_order_bitwise(hip, store1, rng, E, dim, s):
-    """The matrix-core router (more than 8 tokens; both tile sizes, ragged
-    tokens and experts, one and two blocks a chain, waves without chains)
-    gives, bit for bit, the scores of calls of at most 8 tokens."""
+    """Both kernels for more than 8 tokens give, bit for bit, the scores of
+    calls of at most 8 tokens."""
     inter, topk = 128, 4
     cfg, shared, x = _case(rng, E, dim, inter, s, topk, 0, 1.0)
     st = store1(E, dim, inter)
