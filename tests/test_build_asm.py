@@ -1,4 +1,6 @@
-"""Checks on the gfx950 assembly of the GEMM kernels (CPU: hipcc cross-compiles).
+"""Checks on the gfx950 assembly of the kernels with matrix instructions (CPU:
+hipcc cross-compiles): the block-scaled GEMMs of apus_gemm.hip, and the
+plain-weight GEMM and the router of apus_kernels.hip.
 
 A matrix instruction issued while EXEC is narrowed (inside a lane-dependent
 branch) does not read the inactive lanes' operands, so its result is wrong for
@@ -83,6 +85,21 @@ def gemm_asm(tmp_path_factory):
 def test_no_mfma_under_narrowed_exec(gemm_asm):
     assert gemm_asm.count("v_mfma") > 1000          # every schedule was instantiated
     assert _mfma_under_narrowed_exec(gemm_asm) == {}
+
+
+@pytest.fixture(scope="module")
+def kernels_asm(tmp_path_factory):
+    if not os.path.exists(HIPCC) and not shutil.which("hipcc"):
+        pytest.skip("no hipcc")
+    return _asm(os.path.join(CSRC, "apus_kernels.hip"), tmp_path_factory.mktemp("asm"))
+
+
+def test_no_mfma_under_narrowed_exec_kernels(kernels_asm):
+    for name, count in (("apus_wgemm_kernel", 8), ("apus_router_mfma_kernel", 2)):
+        found = [m for m in re.findall(r"^(_Z\d+" + name + r"\S*):", kernels_asm, re.M)]
+        assert len(found) == count, found
+    assert kernels_asm.count("v_mfma") > 100
+    assert _mfma_under_narrowed_exec(kernels_asm) == {}
 
 
 def test_tile_stores_not_serialised(gemm_asm):
