@@ -793,6 +793,12 @@ int moe_pipeline(int E, int dim, int inter, float limit, uint8_t *const *tab,
      * most min(E, nj) experts are small and at most nj / (SMALL + 1) are
      * large, so the launches cover only that many table slots */
     constexpr int SMALL = MOE_SMALL;
+    /* g, u, h and eo lie at multiples of 256 from the workspace, and the SwiGLU
+     * kernels read g and u 16 bytes at a time: refused before the first launch */
+    if (reinterpret_cast<uintptr_t>(w.gm) & 15) {
+        set_err("moe pipeline: the workspace has to be 16-byte aligned");
+        return 1;
+    }
     if (!launched(apus_launch_act_quant(x, dim, nullptr, s, dim, w.xc, w.xs, st), "act_quant"))
         return 1;
     if (rd) {

@@ -18,9 +18,18 @@
  *    GEMMs of many rows, and the routed w1/w3 with SwiGLU at many rows.
  *  - narrow (apus_gemm_narrow_kernel): dense FP8 GEMMs of 9..64 rows.
  *  - stream (apus_gemm_stream_kernel): other grouped shapes.
- * In all of them, every output is one accumulation chain over its 128-groups
- * in a fixed order, so results do not depend on M, on the position of a row
- * within its entry, or on timing.
+ *  - tile (apus_gemm_tile_kernel): other dense GEMMs of more than 8 rows
+ *    (row-major weights, row tables, operands not aligned for the two above).
+ *  - split-K GEMV, grouped GEMV (apus_gemv_split_kernel, apus_gemv_grp_kernel):
+ *    launches of at most 8 rows on tiled weights.
+ * In each of them an output is summed in a fixed order, so its bits do not
+ * depend on timing or on the position of a row within its entry. The order:
+ * one chain over the 128-groups in prefill, block, tile and stream; chains over
+ * parts of K, added in K order, where waves split K (split-K, decode by its
+ * split, narrow: quarters; the GEMVs). Within a schedule it does not depend on
+ * M; a dense row whose batch grows into another schedule can change in its last
+ * bits (64 rows to 65: narrow to block). The routed dispatch asks for one order
+ * (kchain) and gets it from every schedule it uses.
  *
  * Build-time tuning constants (defaults are the measured best on gfx950;
  * -D overrides exist for measurements only): APUS_DEC_WAVES (decode
@@ -2288,7 +2297,6 @@ void apus_launch_grp(const ApusGemmArgs &a, int n_ent, hipStream_t st) {
     else             apus_launch_grp_k<WF, 16>(a, n_ent, st);
 }
 
-/* launch the LDS tile schedule (returns false where it does not apply) */
 /*
  * LDS many-row schedule for the routed MXFP4 experts (grouped launches from
  * the route kernel's work list, MFMA-tiled weights, K 2048 / 4096): one

@@ -881,6 +881,9 @@ __global__ __launch_bounds__(256) void apus_moe_accum_bf16_kernel(
 hipError_t apus_launch_moe_accum_bf16(const uint16_t *eo, const float *wgt, int s, int topk, int dim, float *y,
                                       const float *add_src, float *add_out, hipStream_t st) {
     if (s <= 0) return hipSuccess;
+    if (dim % 8 || ((reinterpret_cast<uintptr_t>(eo) | reinterpret_cast<uintptr_t>(y) |
+                     reinterpret_cast<uintptr_t>(add_src) | reinterpret_cast<uintptr_t>(add_out)) & 15))
+        return hipErrorInvalidValue;
     hipLaunchKernelGGL(apus_moe_accum_bf16_kernel, dim3((dim / 8 + 255) / 256, s), dim3(256), 0, st, eo, wgt, topk,
                        dim, y, add_src, add_out);
     return hipGetLastError();

@@ -194,7 +194,12 @@ int apus_hip_fp8_gemm(const uint8_t *w, const uint8_t *ws,
 /* ---- device-pointer entry points (asynchronous on the backend stream) ----
  * Same semantics as the host versions; all pointers are device pointers.
  * They exist for callers that keep activations in HBM between layers and
- * for measurement with inputs already resident. */
+ * for measurement with inputs already resident.
+ * Alignment: workspaces 16 bytes (the MoE entry points refuse others where
+ * they sort the pairs), other arrays 4 bytes. Arrays that are 16-byte aligned
+ * take the fast schedules; others give the same results, within the GEMM bars,
+ * on slower ones.
+ */
 /* A group holding +-inf gets the scale +inf (as the reference's does) and
  * signed-zero codes for its finite elements; the GEMMs then return NaN for
  * that row (E8M0 255 is NaN on the matrix cores). Non-finite activations are
@@ -210,7 +215,7 @@ int apus_hip_act_quant_dev(const float *x, int M, int K, uint8_t *codes,
  * within a few fp32 ulps of a BF16 rounding boundary. */
 int apus_hip_swiglu_dev(const float *g, const float *u, size_t n, float limit, float *h);
 /* round_out: bit 0 BF16-rounds the outputs; | APUS_HIP_W_TILED for weights
- * in the MFMA-tiled layout (K 2048/4096, O % 128 == 0). */
+ * in the MFMA-tiled layout (K 1024, 2048, 4096 or 8192, O % 128 == 0). */
 int apus_hip_fp4_gemm_dev(const uint8_t *w, const uint8_t *ws,
                           const uint8_t *acodes, const float *as, float *out,
                           int M, int O, int K, int round_out);
@@ -259,7 +264,7 @@ int apus_hip_fp8_linear_dev(const uint8_t *w, const uint8_t *ws,
                             const float *x, float *out, int M, int K, int O,
                             void *workspace);
 /* Either format: wfmt 0 (MXFP4) or 1 (FP8), | APUS_HIP_W_TILED for weights
- * in the MFMA-tiled layout (K 2048/4096, O % 128 == 0). */
+ * in the MFMA-tiled layout (K 1024, 2048, 4096 or 8192, O % 128 == 0). */
 int apus_hip_linear_dev(int wfmt, const uint8_t *w, const uint8_t *ws,
                         const float *x, float *out, int M, int K, int O,
                         void *workspace);
@@ -293,7 +298,8 @@ int      apus_hip_store_get(const ApusHipStore *st, int layer, int eid,
                             const uint8_t *ptrs[6]);
 /* 1 when the store holds its matrices MFMA-tiled. */
 int      apus_hip_store_tiled(const ApusHipStore *st);
-/* Workspace bytes for apus_hip_moe_routed_dev with s tokens x topk. */
+/* Workspace bytes for apus_hip_moe_routed_dev with s tokens x topk (the
+ * workspace 16-byte aligned). */
 size_t   apus_hip_moe_workspace(const ApusHipStore *st, int s, int topk);
 /* Routed dispatch of one layer with everything in HBM: x [s, dim] f32,
  * idx/wgt [s, topk] (device), y [s, dim] f32 (device). Asynchronous. */

@@ -342,3 +342,24 @@ def test_moe_routed_block_schedule(hip, oracle, store, rng, dim):
         if a == 0:
             host = {e: host_expert(oracle, 5, 0, e, E, dim, inter) for e in range(7)}
             stage_check(hip, oracle, st, lambda e: host[e], x[:b], idx[:b], wgt[:b], yp, wsp, inter, [0, 17, 49])
+
+
+def test_moe_routed_workspace_alignment(hip, store, rng):
+    """The sorted dispatch refuses a workspace that is not 16-byte aligned
+    before it launches anything: y and the workspace stay as they were."""
+    E, dim, inter, s, topk = 8, 2048, 2048, 20, 4
+    st = store(1, E, dim, inter)
+    L = hip.lib()
+    hip._check(L.apus_hip_store_fill_random(st, 5), "fill")
+    idx, wgt = topk_routing(rng, s, E, topk)
+    n = L.apus_hip_moe_workspace(st, s, topk)
+    dx, di, dw = (hip.DevBuf.from_array(v) for v in (acts(rng, s, dim), idx, wgt))
+    dy, wsp = (hip.DevBuf.from_array(np.full(k, 0x5A, np.uint8)) for k in (s * dim * 4, n + 16))
+    assert L.apus_hip_moe_routed_dev(st, 0, dx.ptr, di.ptr, dw.ptr, s, topk, 10.0, dy.ptr, wsp.ptr + 8) != 0
+    assert b"16-byte aligned" in L.apus_hip_last_error()
+    hip._check(L.apus_hip_synchronize(), "sync")
+    assert np.all(dy.to_array(np.uint8, (s * dim * 4,)) == 0x5A)
+    assert np.all(wsp.to_array(np.uint8, (n + 16,)) == 0x5A)
+    hip._check(L.apus_hip_moe_routed_dev(st, 0, dx.ptr, di.ptr, dw.ptr, s, topk, 10.0, dy.ptr, wsp.ptr + 16 - wsp.ptr % 16),
+               "aligned")
+    hip._check(L.apus_hip_synchronize(), "sync")
