@@ -1572,11 +1572,15 @@ __device__ __forceinline__ int apus_block_tile_scales(const uint8_t *p) {
 /* tile of workgroup b: each XCD (workgroups are dealt to the 8 XCDs round
  * robin) takes a contiguous band of tiles, ordered in groups of up to 8 row
  * blocks by every column block, so that the tiles running together on an XCD
- * share both operands in its L2 */
+ * share both operands in its L2. Where 8 would leave one or two of few row
+ * blocks, which stream all the weights for themselves, the groups are even (64 x
+ * 128 tiles, FP8, 513 x 3072, 9 row blocks, K 4096 / 8192: 21.8 / 36.2 us in
+ * groups of 8 and 1, 18.5 / 28.7 of 5 and 4) */
 __device__ __forceinline__ void apus_block_tile(int b, int mt, int nt, int &mb, int &nb) {
     const int tiles = mt * nt, per = tiles >> 3, rem = tiles & 7, x = b & 7;
     const int t = x * per + min(x, rem) + (b >> 3);
-    const int grp = t / (8 * nt), g0 = grp * 8, gm = min(8, mt - g0), in = t - grp * 8 * nt;
+    const int gs = mt == 9 || mt == 10 ? 5 : mt == 17 || mt == 18 ? 6 : 8;
+    const int grp = t / (gs * nt), g0 = grp * gs, gm = min(gs, mt - g0), in = t - grp * gs * nt;
     mb = g0 + in % gm;
     nb = in / gm;
 }
@@ -1637,8 +1641,8 @@ bool apus_launch_block_tile(const ApusGemmArgs &a, hipStream_t st) {
     return true;
 }
 
-/* The tile: the largest that still gives most of the 256 CUs a workgroup and
- * pads few rows. A larger tile needs fewer LDS and L2 bytes per MFMA (what
+/* The tile: the largest that still gives most of the 256 CUs a workgroup, pads
+ * few rows and does not leave most CUs idle in its last round. A larger tile needs fewer LDS and L2 bytes per MFMA (what
  * bounds the loop), but a workgroup's time does not shrink when CUs idle.
  * Measured with the act quant, us, [rows, O, K] FP8 unless said (tiles
  * 256 x 128 / 128 x 128 / 64 x 128 / 64 x 64; workgroups of the first / last;
@@ -1651,9 +1655,18 @@ bool apus_launch_block_tile(const ApusGemmArgs &a, hipStream_t st) {
  *   100 x 4096 x 4096      29.1 / 19.6 / 14.8 / 11.9        / 128     15.4
  *   4096 x 4096 x 8192    177.6 / 213.7 / 242.9 / 293.0               254.1
  *   MXFP4 512 x 4096 x 4096  31.8 / 20.1 / 15.2 / 17.4                19.3
- * 64 x 128 runs four stages deep where every CU has one workgroup, three
+ * 64 x 128 runs four stages deep where a CU has one workgroup at most, three
  * (two workgroups a CU) past that: 18.4 / 18.9 at 256 workgroups, 27.2 / 24.3
- * at 1280. */
+ * at 1280. From 129 workgroups of 64 x 128 on it is ahead of twice as many of 64
+ * x 64, which no longer fit one to a CU (700 x 2048 x 8192, 176, 29.6 / 33.6; 200
+ * x 4096 x 4096, 128, 18.1 / 14.7).
+ * The larger tiles run one workgroup a CU, so tiles past a multiple of 256 cost
+ * a round of their own; 64 x 128 runs on. Up to three rounds, with the last at
+ * most about half full, that is worth more than the larger tile (before / larger
+ * tile / 64 x 128): FP8 1025 x 4096 x 1024 (288 of 128 x 128) 19.3 / 20.7 / 17.9, 768 x
+ * 8192 x 4096 (384) 47.9 / 45.5 / 41.2, 1280 x 8192 x 8192 (640) 137.3 / 127.3 /
+ * 112.9; MXFP4 1200 x 4096 x 4096 (320) 48.0 / 41.4 / 35.9. With 400: FP8 1280 x
+ * 5120 x 8192 the larger tile is 11 % ahead. */
 template <int WF, int NQ>
 bool apus_launch_block(const ApusGemmArgs &a, hipStream_t st) {
     const int M = a.ent0.M;
@@ -1662,11 +1675,13 @@ bool apus_launch_block(const ApusGemmArgs &a, hipStream_t st) {
         const size_t padded = (size_t)((M + bm - 1) / bm) * bm;
         return tiles(bm, bn) >= 224 && padded * 6 <= (size_t)M * 7;
     };
-    if (fits(256, 128)) return apus_launch_block_tile<WF, NQ, 256, 128, 4, 2, 3>(a, st);
-    if (fits(128, 128)) return apus_launch_block_tile<WF, NQ, 128, 128, 2, 4, 4>(a, st);
+    const size_t t128 = tiles(128, 128), last = t128 % 256;
+    const bool ragged = t128 > 256 && t128 <= 768 && last > 0 && last <= 136;
+    if (!ragged && fits(256, 128)) return apus_launch_block_tile<WF, NQ, 256, 128, 4, 2, 3>(a, st);
+    if (!ragged && fits(128, 128)) return apus_launch_block_tile<WF, NQ, 128, 128, 2, 4, 4>(a, st);
     const size_t t = tiles(64, 128);
     if (t > 256) return apus_launch_block_tile<WF, NQ, 64, 128, 2, 2, 3>(a, st);
-    if (t >= 224) return apus_launch_block_tile<WF, NQ, 64, 128, 2, 2, 4>(a, st);
+    if (t > 128) return apus_launch_block_tile<WF, NQ, 64, 128, 2, 2, 4>(a, st);
     return apus_launch_block_tile<WF, NQ, 64, 64, 2, 2, 4>(a, st);
 }
 

@@ -66,7 +66,10 @@ def gemm_rows(hip, fmt, w, ws, c, s, round_out=0):
 @pytest.mark.parametrize("fmt,M,O,K", [
     (1, 500, 14336, 1024), (0, 449, 14336, 1024),      # 256 x 128 tiles
     (1, 120, 28672, 1024), (0, 380, 10240, 2048),      # 128 x 128
-    (1, 65, 16384, 1024), (1, 200, 8192, 2048),        # 64 x 128, 256 workgroups; more
+    (1, 65, 16384, 1024), (1, 200, 8192, 2048),        # 64 x 128, 256 workgroups
+    (0, 150, 6144, 1024), (1, 129, 5760, 2048), (1, 300, 8192, 1024),   # 64 x 128: 144, 135; more than 256
+    (1, 300, 12288, 1024), (0, 300, 12288, 1024),      # 64 x 128 for 288 tiles of 128 x 128
+    (1, 520, 1536, 1024), (0, 1040, 384, 1024), (1, 577, 2048, 1024),   # even groups of row blocks: 9, 17, 10
     (1, 66, 128, 8192), (0, 9, 128, 1024), (1, 129, 384, 4096), (0, 64, 256, 4096), (0, 70, 128, 2048),  # 64 x 64
     (1, 1000, 1024, 4096),
 ])
