@@ -1355,7 +1355,7 @@ __global__ __launch_bounds__(64 * NW) void apus_gemm_tile_kernel(ApusGemmArgs ar
  * tiled layout), and from LDS into a second set of fragment registers one
  * step ahead of the MFMAs, so a slot is free for its next stage as soon as
  * the barrier after that read. Scales come per four groups (16 bytes a row),
- * in a ring of two. Nothing in the loop but these loads uses vmcnt: mixed with
+ * in a ring of two, or all at the start (SUP). Nothing in the loop but these loads uses vmcnt: mixed with
  * loads into registers, the compiler would drain all of them at each use.
  * The weights are the MFMA's first operand, so a lane ends up with four
  * consecutive outputs of one row. Every output is one chain over the
@@ -1369,9 +1369,18 @@ struct ApusBlk {
     static constexpr int FB = FP4 ? 1024 : 2048;             /* bytes of a weight fragment */
     static constexpr int AB = BM * 128, STB = AB + BN / 16 * FB;
     static constexpr int LA = BM / 8, LPW = STB / 1024 / NW; /* loads of a stage: activations; per wave */
-    static constexpr int SI = BM / 64 + (FP4 ? BN / 64 : 0), SPW = (SI + NW - 1) / NW;
+    /* FP8, 64 rows: every activation scale of the block comes at the start, where
+     * LDS has room beside as many workgroups a CU as without: four groups at a
+     * time are 64 cache lines a load, in every wave, beside the stages' 192 (512 x
+     * 4096 x 4096, a fresh weight copy per launch 17.8 -> 16.75 us, the same one
+     * again 14.4 -> 14.7; with the act quant before it 22.9 -> 21.8, 19.5 -> 19.1) */
+    static constexpr bool SUP = !FP4 && BM == 64 && (NST == 4 && BN == 128 ? true : NST * STB + BM * NQ * 4 <= 80 * 1024);
+    static constexpr int SC = NQ >= 32 ? 8 : NQ / 4, SUI = BM * NQ / 256; /* 16-byte chunks of a row in a run; loads */
+    static constexpr int SI = SUP ? 0 : BM / 64 + (FP4 ? BN / 64 : 0), SPW = (SI + NW - 1) / NW;
     static constexpr int SB = SI * 1024;                     /* bytes of a scale block (four groups) */
-    static constexpr int LDS = NST * STB + 2 * SB;
+    static constexpr int LDS = NST * STB + (SUP ? SUI * 1024 : 2 * SB);
+    /* chunk c of row i is in slot c ^ sswz(i) of its SC: 16 rows' reads meet no bank twice */
+    __device__ static int sswz(int i) { return i / (16 / SC) % SC; }
     static_assert(STB / 1024 % NW == 0 && NST >= 2 && NST <= 4 && NQ % 4 == 0 && BM % 64 == 0 && BN % 64 == 0 &&
                       LDS <= 160 * 1024,
                   "block shape");
@@ -1414,11 +1423,20 @@ __device__ __forceinline__ void apus_block_loop(uint8_t *lds, const uint8_t *aco
             voff[u] = lane * 16;
         }
     }
-    const uint8_t *ssrc[B::SPW];
-    unsigned sdst[B::SPW], sstep[B::SPW];
+    if constexpr (B::SUP) {
+        constexpr int UW = (B::SUI + B::NW - 1) / B::NW;
+#pragma unroll
+        for (int u = 0; u < UW; ++u) {
+            const int ii = (wave * UW + u) % B::SUI, p = 64 * ii + lane;     /* spare waves repeat a load */
+            const int run = p / (B::BM * B::SC), i = p / B::SC % B::BM, c = p % B::SC ^ B::sswz(i);
+            apus_g2lds16(ascale + (size_t)row(i) * NQ + run * 32 + 4 * c, lbase + NST * STB + ii * 1024);
+        }
+    }
+    const uint8_t *ssrc[B::SPW + 1];
+    unsigned sdst[B::SPW + 1], sstep[B::SPW + 1];
 #pragma unroll
     for (int u = 0; u < B::SPW; ++u) {
-        const int ii = (wave * B::SPW + u) % B::SI;          /* spare waves repeat a load */
+        const int ii = (wave * B::SPW + u) % (B::SI + B::SUP);          /* spare waves repeat a load */
         if (ii < B::BM / 64) {
             ssrc[u] = reinterpret_cast<const uint8_t *>(ascale + (size_t)row(64 * ii + lane) * NQ);
             sstep[u] = 16;
@@ -1465,7 +1483,12 @@ __device__ __forceinline__ void apus_block_loop(uint8_t *lds, const uint8_t *aco
             const apus_v4u lo = *reinterpret_cast<const apus_v4u *>(p + ((g ^ sw) << 4));
             const apus_v4u hi = *reinterpret_cast<const apus_v4u *>(p + (((4 + g) ^ sw) << 4));
             f.a[t] = apus_v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-            f.sa[t] = *reinterpret_cast<const float *>(sc + ar * 16 + 4 * qb);
+            if constexpr (B::SUP)
+                f.sa[t] = *reinterpret_cast<const float *>(lds + NST * STB + (q >> 5) * (B::BM * 128) +
+                                                           (ar * B::SC + (((q >> 2) & (B::SC - 1)) ^ B::sswz(ar))) * 16 +
+                                                           4 * qb);
+            else
+                f.sa[t] = *reinterpret_cast<const float *>(sc + ar * 16 + 4 * qb);
         }
     };
 #pragma unroll
@@ -1660,26 +1683,35 @@ bool apus_launch_block_tile(const ApusGemmArgs &a, hipStream_t st) {
  * at 1280. From 129 workgroups of 64 x 128 on it is ahead of twice as many of 64
  * x 64, which no longer fit one to a CU (700 x 2048 x 8192, 176, 29.6 / 33.6; 200
  * x 4096 x 4096, 128, 18.1 / 14.7).
+ * Between 257 and 447 workgroups of 64 x 128 some CUs have two and the others
+ * wait; half as many of 128 x 128, one a CU, are done sooner where a weight row
+ * has 4 KB or more (64 x 128 / 128 x 128, a fresh weight copy per launch, then the
+ * same one again): FP8 640 x 4096 x 8192 60.8 / 50.0, 45.3 / 40.2; 640 x 4096 x
+ * 4096 30.5 / 29.6, 26.1 / 26.2; MXFP4 576 x 4096 x 8192 39.5 / 35.7, 36.1 / 34.4;
+ * but FP8 2048 x 1536 x 2048 20.9 / 22.2, MXFP4 700 x 4096 x 1024 12.1 / 12.5, and
+ * with 128 of 128 x 128, FP8 4096 x 512 x 4096, 33.0 / 38.2.
  * The larger tiles run one workgroup a CU, so tiles past a multiple of 256 cost
  * a round of their own; 64 x 128 runs on. Up to three rounds, with the last at
- * most about half full, that is worth more than the larger tile (before / larger
- * tile / 64 x 128): FP8 1025 x 4096 x 1024 (288 of 128 x 128) 19.3 / 20.7 / 17.9, 768 x
- * 8192 x 4096 (384) 47.9 / 45.5 / 41.2, 1280 x 8192 x 8192 (640) 137.3 / 127.3 /
- * 112.9; MXFP4 1200 x 4096 x 4096 (320) 48.0 / 41.4 / 35.9. With 400: FP8 1280 x
- * 5120 x 8192 the larger tile is 11 % ahead. */
+ * most about half full, that is worth more than the larger tile (larger tile / 64
+ * x 128): FP8 1025 x 4096 x 1024 (288 of 128 x 128) 20.7 / 17.9, 768 x 8192 x 4096
+ * (384) 45.5 / 41.2, 1280 x 8192 x 8192 (640) 127.3 / 112.9; MXFP4 1200 x 4096 x
+ * 4096 (320) 41.4 / 35.9. With 400: FP8 1280 x 5120 x 8192 the larger tile is 11 %
+ * ahead; with 384 and rows of 8 KB, a fresh weight copy per launch, 8 % (700 x 8192 x
+ * 8192). */
 template <int WF, int NQ>
 bool apus_launch_block(const ApusGemmArgs &a, hipStream_t st) {
     const int M = a.ent0.M;
     auto tiles = [&](int bm, int bn) { return (size_t)((M + bm - 1) / bm) * (a.O / bn); };
-    auto fits = [&](int bm, int bn) {
+    auto fits = [&](int bm, size_t least) {
         const size_t padded = (size_t)((M + bm - 1) / bm) * bm;
-        return tiles(bm, bn) >= 224 && padded * 6 <= (size_t)M * 7;
+        return tiles(bm, 128) >= least && padded * 6 <= (size_t)M * 7;
     };
-    const size_t t128 = tiles(128, 128), last = t128 % 256;
-    const bool ragged = t128 > 256 && t128 <= 768 && last > 0 && last <= 136;
-    if (!ragged && fits(256, 128)) return apus_launch_block_tile<WF, NQ, 256, 128, 4, 2, 3>(a, st);
-    if (!ragged && fits(128, 128)) return apus_launch_block_tile<WF, NQ, 128, 128, 2, 4, 4>(a, st);
-    const size_t t = tiles(64, 128);
+    constexpr int WB = NQ * (WF == APUS_W_FP4 ? 64 : 128);   /* bytes of a weight row */
+    const size_t t128 = tiles(128, 128), last = t128 % 256, t = tiles(64, 128);
+    const bool ragged = t128 > 256 && t128 <= 768 && last > 0 && last <= (WB >= 8192 ? 104 : 136);
+    if (!ragged && fits(256, 224)) return apus_launch_block_tile<WF, NQ, 256, 128, 4, 2, 3>(a, st);
+    if (!ragged && fits(128, WB >= 4096 && t > 256 ? 129 : 224))
+        return apus_launch_block_tile<WF, NQ, 128, 128, 2, 4, 4>(a, st);
     if (t > 256) return apus_launch_block_tile<WF, NQ, 64, 128, 2, 2, 3>(a, st);
     if (t > 128) return apus_launch_block_tile<WF, NQ, 64, 128, 2, 2, 4>(a, st);
     return apus_launch_block_tile<WF, NQ, 64, 64, 2, 2, 4>(a, st);
