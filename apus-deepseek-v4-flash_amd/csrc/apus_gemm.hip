@@ -1379,7 +1379,7 @@ struct ApusBlk {
     static constexpr int SI = SUP ? 0 : BM / 64 + (FP4 ? BN / 64 : 0), SPW = (SI + NW - 1) / NW;
     static constexpr int SB = SI * 1024;                     /* bytes of a scale block (four groups) */
     static constexpr int LDS = NST * STB + (SUP ? SUI * 1024 : 2 * SB);
-    /* chunk c of row i is in slot c ^ sswz(i) of its SC: 16 rows' reads meet no bank twice */
+    /* chunk c of row i is in slot c ^ sswz(i) of its SC: of 16 rows, two a bank */
     __device__ static int sswz(int i) { return i / (16 / SC) % SC; }
     static_assert(STB / 1024 % NW == 0 && NST >= 2 && NST <= 4 && NQ % 4 == 0 && BM % 64 == 0 && BN % 64 == 0 &&
                       LDS <= 160 * 1024,
@@ -1665,8 +1665,11 @@ bool apus_launch_block_tile(const ApusGemmArgs &a, hipStream_t st) {
 }
 
 /* The tile: the largest that still gives most of the 256 CUs a workgroup, pads
- * few rows and does not leave most CUs idle in its last round. A larger tile needs fewer LDS and L2 bytes per MFMA (what
- * bounds the loop), but a workgroup's time does not shrink when CUs idle.
+ * few rows and does not leave most CUs idle in its last round. A larger tile needs fewer LDS and L2 bytes and fewer
+ * barriers per MFMA, but a workgroup's time does not shrink when CUs idle. What
+ * bounds the loop is waiting: by the counters the matrix cores are busy 20-28 % of
+ * the cycles, LDS reads 13-28 %; a step's stage, barrier and fragment reads come
+ * one after the other for the one or two waves of a SIMD.
  * Measured with the act quant, us, [rows, O, K] FP8 unless said (tiles
  * 256 x 128 / 128 x 128 / 64 x 128 / 64 x 64; workgroups of the first / last;
  * before):
@@ -1730,8 +1733,9 @@ bool apus_launch_block(const ApusGemmArgs &a, hipStream_t st) {
  * 4096 tokens x top-6, 256 experts, Zipf token ids: 690 us + 90 for that
  * kernel -> 668 (1.23 PFLOP/s of the rows asked for, 77 % of those multiplied);
  * 512 tokens, Zipf experts, 125 + 15 -> 135 (+ 8 for the few-row experts' rows).
- * Bound by LDS bandwidth (128 KB a step of 128 rows) and, one workgroup a CU,
- * by its start and end; without MFMAs it runs 596 us, without staging 521.
+ * Matrix cores busy 33 % of its cycles, LDS 24 %: the rest is waiting, for a
+ * step's stage and barrier and, one workgroup a CU, at its start and end;
+ * without MFMAs it runs 596 us, without staging 521.
  * w2 on the same loop (64 rows, its four chains) ran 477 us against 450 for the
  * resident-activation schedule at 4096 tokens, 104 against 80 at 512: not kept.
  */

@@ -1078,7 +1078,9 @@ __global__ __launch_bounds__(256) void apus_head_kernel(const uint16_t *__restri
  *
  * 512 x 1024 x 4096: BF16 weights 137 -> 21-25 us (175-200 TFLOP/s), FP32
  * weights 132 -> 53 us (half the fp32 MFMA rate). Bound by the L2 -> CU stream of
- * both operands (1 MB a CU) and the splitting of x on the vector units. */
+ * both operands (1 MB a CU), the splitting of x on the vector units, and the wait
+ * for every load in flight that the compiler puts before the reads of a slot
+ * (matrix cores 25 %, LDS 18 % of the cycles busy). */
 typedef __bf16 apus_v8bf __attribute__((ext_vector_type(8)));
 
 /* BF16 pieces of 8 fp32 values, nearest-even (one packed conversion per two
